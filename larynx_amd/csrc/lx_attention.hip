@@ -376,7 +376,7 @@ __global__ __launch_bounds__(64 * QS * KS) void attn_flash_kernel(
     const floatx16& keep = ks == 0 ? o0 : o1;
     const int qi = q0 + r;
     if (qi < Tq) {
-      float* orow = o + ((long)b * Tq + qi) * ldo + head * kHD + ks * 32 + h * 4;
+      const int col = head * kHD + ks * 32 + h * 4;
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         floatx4 w;
@@ -386,7 +386,10 @@ __global__ __launch_bounds__(64 * QS * KS) void attn_flash_kernel(
           const float mine = keep[i] * a_s, other = part[i * 64 + lane] * a_o;
           w[e] = (ks == 0 ? mine + other : other + mine) * inv;
         }
-        store_o4(orow + g * 8, w, opk);
+        if (opk < LX_ACT_FRAG2)
+          store_o4(o + ((long)b * Tq + qi) * ldo + col + g * 8, w, opk);
+        else
+          act_store4(o, ldo, b * Tq + qi, col + g * 8, w, opk);
       }
     }
     return;
@@ -445,8 +448,11 @@ __global__ __launch_bounds__(64 * QS * KS) void attn_flash_kernel(
     const int qi = qt0 + row;
     if (qi < Tq) {
       const float* src = otile + (row >> 5) * (32 * kLD) + (row & 31) * kLD + c;
-      store_o4(o + ((long)b * Tq + qi) * ldo + head * kHD + c,
-               *reinterpret_cast<const floatx4*>(src), opk);
+      const floatx4 w = *reinterpret_cast<const floatx4*>(src);
+      if (opk < LX_ACT_FRAG2)
+        store_o4(o + ((long)b * Tq + qi) * ldo + head * kHD + c, w, opk);
+      else
+        act_store4(o, ldo, b * Tq + qi, head * kHD + c, w, opk);
     }
   }
 }
@@ -951,7 +957,7 @@ __global__ __launch_bounds__(64 * QS * KS) void attn_bx_kernel(
     const floatx16& keep = ks == 0 ? o0 : o1;
     const int qi = q0 + r;
     if (qi < Tq) {
-      float* orow = o + ((long)b * Tq + qi) * ldo + head * kHD + ks * 32 + h * 4;
+      const int col = head * kHD + ks * 32 + h * 4;
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         floatx4 w;
@@ -961,7 +967,10 @@ __global__ __launch_bounds__(64 * QS * KS) void attn_bx_kernel(
           const float mine = keep[i] * a_s, other = part[i * 64 + lane] * a_o;
           w[e] = (ks == 0 ? mine + other : other + mine) * inv;
         }
-        store_o4(orow + g * 8, w, opk);
+        if (opk < LX_ACT_FRAG2)
+          store_o4(o + ((long)b * Tq + qi) * ldo + col + g * 8, w, opk);
+        else
+          act_store4(o, ldo, b * Tq + qi, col + g * 8, w, opk);
       }
     }
     return;
@@ -1020,8 +1029,11 @@ __global__ __launch_bounds__(64 * QS * KS) void attn_bx_kernel(
     const int qi = qt0 + row;
     if (qi < Tq) {
       const float* src = otile + (row >> 5) * (32 * kLD) + (row & 31) * kLD + c;
-      store_o4(o + ((long)b * Tq + qi) * ldo + head * kHD + c,
-               *reinterpret_cast<const floatx4*>(src), opk);
+      const floatx4 w = *reinterpret_cast<const floatx4*>(src);
+      if (opk < LX_ACT_FRAG2)
+        store_o4(o + ((long)b * Tq + qi) * ldo + head * kHD + c, w, opk);
+      else
+        act_store4(o, ldo, b * Tq + qi, head * kHD + c, w, opk);
     }
   }
 }
@@ -1045,7 +1057,7 @@ bool attention_takes_packed_kv(int B, int Tq, int n_heads, int products) {
 
 int attention(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, float* o,
               int ldo, int B, int Tq, int Tk, int n_heads, int n_kv_heads, int head_dim,
-              float scale, int causal, int q_offset, int products, int out_packed,
+              float scale, int causal, int q_offset, int products, int out_form,
               hipStream_t stream, int kv_packed) {
   LX_REQUIRE(products == 3 || products == 6, "attention: %d products (3 or 6)", products);
   LX_REQUIRE(q && k && v && o, "attention: null pointer");
@@ -1060,6 +1072,8 @@ int attention(const float* q, int ldq, const float* k, int ldk, const float* v, 
                  ((uintptr_t)q | (uintptr_t)k | (uintptr_t)o) % 16 == 0,
              "attention: q/k/o rows must be 16-byte aligned");
   LX_REQUIRE(ldv % 4 == 0 && (uintptr_t)v % 16 == 0, "attention: v rows must be 16-byte aligned");
+  LX_REQUIRE(out_form < LX_ACT_FRAG2 || ldo % 16 == 0, "attention: fragment order needs ldo %% 16");
+  LX_REQUIRE((long)B * Tq < (1L << 31), "attention: too many rows");
   LX_REQUIRE(q_offset >= 0, "attention: q_offset < 0");
   if (causal) LX_REQUIRE(q_offset + Tq <= Tk, "attention: causal needs q_offset + Tq <= Tk");
   const int rep = n_heads / n_kv_heads;
@@ -1135,7 +1149,7 @@ int attention(const float* q, int ldq, const float* k, int ldk, const float* v, 
   LX_REQUIRE(nwg < (1L << 31), "attention: %ld workgroups exceed the grid limit", nwg);
   hipLaunchKernelGGL(kern, dim3((unsigned)nwg), dim3(threads), lds, stream, q, ldq, k, ldk, v, ldv,
                      o, ldo, Tq, Tk, n_heads, rep, scale * log2e, causal, q_offset,
-                     out_packed ? 1 : 0);
+                     out_form);
   return check_launch("attn_flash_kernel");
 }
 
@@ -1157,5 +1171,5 @@ extern "C" int lx_attention_np_f32(const float* q, int ldq, const float* k, int 
                                    int causal, int q_offset, int products, int out_packed,
                                    int kv_packed, hipStream_t stream) {
   return attention(q, ldq, k, ldk, v, ldv, o, ldo, B, Tq, Tk, n_heads, n_kv_heads, head_dim,
-                   scale, causal, q_offset, products, out_packed, stream, kv_packed);
+                   scale, causal, q_offset, products, out_packed ? LX_ACT_PACKED : LX_ACT_F32, stream, kv_packed);
 }

@@ -39,6 +39,13 @@ constexpr int kSolveChunk = 16;    // solve steps whose modulations one GEMV com
 // whose sum is folded into the next modulated LayerNorm: at B * T = 1000 their
 // 64-row tiles number 128, half the CUs.
 constexpr int kPartialRows = 1024;
+// Up to this many rows the block runs on the fragment-operand GEMMs (linear_fs)
+// with three and with six products.  One evaluation at B = 2: T = 24 2014 -> 1317
+// us, T = 74 1985 -> 1489, T = 160 2188 -> 1845, T = 256 2207 -> 2066 (T = 300 2368 /
+// 2389: even, and the larger launches keep the split tail); six products T = 24
+// 2413 -> 1622, T = 160 2573 -> 2445, T = 211 (422 rows) slower.
+constexpr int kFragRows3 = 512;
+constexpr int kFragRows6 = 320;
 
 }  // namespace
 
@@ -166,26 +173,32 @@ int forward_core(lx_dit* m, const float* x, long x_bstride, const float* mu, con
     const float* gate = nullptr;
   } pend;
   bool pending = false;
-  const bool partial = m->frag && rows <= kPartialRows && D % 128 == 0 && m->F % 128 == 0;
-  // With three products the block's activations (the modulated LayerNorms'
-  // output, attention's output, FF0's GELU output) pass to the projections
-  // that read them as two-part packed rows: each producer splits its output
-  // once, with the roundings the GEMM would apply (bit-identical results),
-  // instead of every column tile of the consumer splitting it again.
-  const bool pk = m->frag && m->products == 3;
-  auto adaln = [&](const float* shift, const float* scale, float* y, bool packed) -> int {
-    if (!pending && !packed)
+  const bool fs = m->frag && rows <= (m->products == 3 ? kFragRows3 : kFragRows6);
+  const bool partial = m->frag && !fs && rows <= kPartialRows;
+  // Up to kFragRows* rows every GEMM input of the block (the modulated
+  // LayerNorms' output, attention's output, FF0's GELU output) is written by its
+  // producer in fragment order, two parts for three products and three for six,
+  // and the residual goes in by the out / FF2 epilogues.  Past them three products
+  // take two-part packed rows: each producer splits its output once, with the
+  // roundings the GEMM would apply (bit-identical results), instead of every
+  // column tile of the consumer splitting it again.
+  const bool pk = m->frag && !fs && m->products == 3;
+  const int form = fs ? (m->products == 3 ? LX_ACT_FRAG2 : LX_ACT_FRAG3)
+                      : pk ? LX_ACT_PACKED : LX_ACT_F32;
+  auto adaln = [&](const float* shift, const float* scale, float* y, int out_form) -> int {
+    if (!pending && out_form == LX_ACT_F32)
       return lx_adaln_modulate_f32(m->h, shift, scale, NA, y, B, T, D, kLnEps, s);
     const int S = pending ? 2 : 0;
     pending = false;
     return adaln_resid(m->h, S ? m->Rws : nullptr, S, (long)rows * D, S ? pend.bias : nullptr,
                        S ? pend.gate : nullptr, NA, shift, scale, NA, y, B, T, D, kLnEps,
-                       packed ? 1 : 0, s);
+                       out_form, s);
   };
   // K and V leave the QKV projection packed too where attention runs on the
   // three-product split kernel (it then stages them without splitting; q
   // stays fp32: attention scales it before its own split).
-  const bool pk_kv = pk && attention_takes_packed_kv(B, T, m->heads, 3);
+  const bool pk_kv =
+      m->frag && m->products == 3 && attention_takes_packed_kv(B, T, m->heads, 3);
   // Every projection on the fragment-order GEMM asks for the split tail: it
   // applies where the launch's tiles number between one and two per CU (T = 500:
   // the QKV projection's 384 tiles run 256 whole and 128 in two k ranges).
@@ -193,6 +206,22 @@ int forward_core(lx_dit* m, const float* x, long x_bstride, const float* mu, con
                   float* y, int ldy, int N, int K, const lx_epilogue* epi,
                   bool pack_out = false, int pack_from = 0) -> int {
     if (!m->frag) return lx_linear_f32(x, ldx, W, bias, y, ldy, rows, N, K, epi, s);
+    if (fs) {
+      FsLinear f;
+      f.A = x;
+      f.Wf = Wf;
+      f.bias = bias;
+      f.epi = epi;
+      f.out = !pack_out ? FS_OUT_F32 : epi->kind == LX_EPI_ROPE_PARTIAL ? FS_OUT_PACKED : FS_OUT_FRAG;
+      f.Y = y;
+      f.ldy = ldy;
+      f.M = rows;
+      f.N = N;
+      f.K = K;
+      f.products = m->products;
+      f.pack_from = pack_from;
+      return linear_fs(f, s);
+    }
     lx_linear_bx g{};
     if (m->qkv_ws) {
       g.split_tail = 1;
@@ -268,7 +297,7 @@ int forward_core(lx_dit* m, const float* x, long x_bstride, const float* mu, con
     const float* w2 = m->frag ? nullptr : m->ff0_w[i];
     const float* w3 = m->frag ? nullptr : m->ff2_w[i];
 
-    LX_TRY(adaln(shift_msa, scale_msa, m->xn, pk));
+    LX_TRY(adaln(shift_msa, scale_msa, m->xn, form));
     lx_epilogue rope{};
     rope.kind = LX_EPI_ROPE_PARTIAL;
     rope.rows_per_batch = T;
@@ -281,10 +310,10 @@ int forward_core(lx_dit* m, const float* x, long x_bstride, const float* mu, con
                 /*pack_from*/ D));
     LX_TRY(attention(m->qkv, 3 * D, m->qkv + D, 3 * D, m->qkv + 2 * D, 3 * D, m->att, D, B, T,
                      T, m->heads, m->heads, m->hd, 1.0f / std::sqrt((float)m->hd), 0, 0,
-                     m->products, pk ? 1 : 0, s, pk_kv ? 1 : 0));
+                     m->products, form, s, pk_kv ? 1 : 0));
     LX_TRY(proj_gated(m->att, D, wf1, w1, m->out_b[i], gate_msa, D));
 
-    LX_TRY(adaln(shift_mlp, scale_mlp, m->xn, pk));
+    LX_TRY(adaln(shift_mlp, scale_mlp, m->xn, form));
     lx_epilogue gelu{};
     gelu.kind = LX_EPI_GELU_TANH;
     LX_TRY(proj(m->xn, D, wf2, w2, m->ff0_b[i], m->ff, m->F, m->F, D, &gelu, /*pack_out*/ true));
@@ -301,7 +330,7 @@ int forward_core(lx_dit* m, const float* x, long x_bstride, const float* mu, con
   }
   // norm_out (AdaLayerNormZero_Final): chunk order scale, shift (src/flow/dit.cpp:134-135).
   const float* ef = emb + (long)m->depth * 6 * D;
-  LX_TRY(adaln(/*shift*/ ef + D, /*scale*/ ef, m->xn, /*packed*/ false));
+  LX_TRY(adaln(/*shift*/ ef + D, /*scale*/ ef, m->xn, LX_ACT_F32));
   if (m->cap.norm_out)
     (void)hipMemcpyAsync(m->cap.norm_out, m->xn, sizeof(float) * rows * D, hipMemcpyDeviceToDevice,
                          s);
@@ -399,10 +428,12 @@ extern "C" int lx_dit_create(const lx_dit_weights* w, int B, int max_T, lx_dit**
   m->xe = A(rows * D);
   m->c1 = A(rows * D);
   m->h = A(rows * D);
-  m->xn = A(rows * D);
+  // (fragment order, up to kFragRows3 rows, takes half as much again)
+  const size_t frows = std::min<size_t>(rows, kFragRows3);
+  m->xn = A(std::max(rows * D, act_floats(frows, D)));
   m->qkv = A(rows * 3 * D);
-  m->att = A(rows * D);
-  m->ff = A(rows * F);
+  m->att = A(std::max(rows * D, act_floats(frows, D)));
+  m->ff = A(std::max(rows * F, act_floats(frows, F)));
   m->P = A(rows * mel);
   m->Pws = A(rows * mel * kProjSplitMax);
   m->Rws = m->frag ? A((size_t)2 * std::min<size_t>(rows, kPartialRows) * D) : nullptr;

@@ -4,6 +4,7 @@
 #pragma once
 
 #include "lx_common.hpp"
+#include "lx_internal.hpp"
 
 namespace lx {
 
@@ -38,6 +39,45 @@ __device__ __forceinline__ uintx4_t pack2_bf16(floatx4 v) {
   const bf16x4_t x1 = __builtin_convertvector(v - bf16x4_back(x0), bf16x4_t);
   const uintx2_t u0 = __builtin_bit_cast(uintx2_t, x0), u1 = __builtin_bit_cast(uintx2_t, x1);
   return uintx4_t{u0[0], u0[1], u1[0], u1[1]};
+}
+
+// Fragment-order activations: a (rows, K) matrix as the A operand of the
+// split-operand GEMMs on v_mfma_f32_32x32x16_bf16, written once by its producer.
+// Per 32-row block, 16-wide k step and bf16 part (NPL = 2 or 3 of them) the 64
+// lanes' 16-byte fragments are one contiguous 1 KB: lane l holds row l % 32,
+// k = (l / 32) * 8 .. + 7.  Rows past the last are never written; they only
+// reach output rows that are not stored.
+__device__ __forceinline__ long frag_index(int row, int col, int nks, int npl) {
+  return ((long)(row >> 5) * nks + (col >> 4)) * npl * 512 +
+         ((row & 31) + ((col >> 3) & 1) * 32) * 8 + (col & 7);
+}
+// Columns col .. col + 3 (col % 4 == 0) of a row.  Contraction off as in pack2_bf16.
+template <int NPL>
+__device__ __forceinline__ void frag_store4(__bf16* base, int row, int col, int nks, floatx4 v) {
+#pragma clang fp contract(off)
+  __bf16* p = base + frag_index(row, col, nks, NPL);
+  const bf16x4_t x0 = __builtin_convertvector(v, bf16x4_t);
+  const floatx4 r = v - bf16x4_back(x0);
+  const bf16x4_t x1 = __builtin_convertvector(r, bf16x4_t);
+  *reinterpret_cast<bf16x4_t*>(p) = x0;
+  *reinterpret_cast<bf16x4_t*>(p + 512) = x1;
+  if (NPL == 3)
+    *reinterpret_cast<bf16x4_t*>(p + 1024) =
+        __builtin_convertvector(r - bf16x4_back(x1), bf16x4_t);
+}
+
+// Columns col .. col + 3 of a row of an activation in one of the forms LX_ACT_*
+// (ld: the fp32 row stride; fragment order: the row width).
+__device__ __forceinline__ void act_store4(float* base, long ld, int row, int col, floatx4 v,
+                                           int form) {
+  if (form == LX_ACT_F32)
+    *reinterpret_cast<floatx4*>(base + row * ld + col) = v;
+  else if (form == LX_ACT_PACKED)
+    *reinterpret_cast<uintx4_t*>(base + row * ld + col) = pack2_bf16(v);
+  else if (form == LX_ACT_FRAG2)
+    frag_store4<2>(reinterpret_cast<__bf16*>(base), row, col, (int)(ld >> 4), v);
+  else
+    frag_store4<3>(reinterpret_cast<__bf16*>(base), row, col, (int)(ld >> 4), v);
 }
 
 __device__ __forceinline__ void rotate_pair(float& x0, float& x1, float ang) {

@@ -8,6 +8,12 @@
 
 namespace lx {
 
+// Output form of an activation producer: fp32 rows, two-part packed rows
+// (pack2_bf16), or fragment order with two or three bf16 parts (frag_store4).
+enum { LX_ACT_F32 = 0, LX_ACT_PACKED = 1, LX_ACT_FRAG2 = 2, LX_ACT_FRAG3 = 3 };
+// Floats that hold a (rows, K) activation in any form.
+inline size_t act_floats(size_t rows, size_t K) { return (rows + 31) / 32 * 32 * K * 3 / 2; }
+
 // Device allocations of a composite object (lx_dit, lx_qwen2, lx_flow), made
 // at create time and released together when the object is destroyed.
 struct Arena {
@@ -82,6 +88,8 @@ int conv_weight_pack(const float* w, float* wp, int C, int G, int K, hipStream_t
 
 // Iota: p[i] = i for i < n.
 int iota_i32(int* p, int n, hipStream_t stream);
+// tab[p * 64 + i] = cos, tab[p * 64 + 32 + i] = sin of fp32(p) * inv_freq[i], i < 32, p < n.
+int rope_table(const float* inv_freq, int n, float* tab, hipStream_t stream);
 // Fill n floats with value.
 int fill_f32(float* p, long n, float value, hipStream_t stream);
 
@@ -119,10 +127,11 @@ int linear_split(const float* x, int ldx, const void* Wp, const float* bias, flo
 // Scratch floats a split tail of this shape uses (0: none) and its tail tiles.
 size_t split_tail_ws_floats(int M, int N, int K, int* tail_tiles);
 // x[m, :] += sum_s ws[s][m, :] (+ bias); then, if norm_w, hn[m, :] =
-// RMSNorm(x[m, :]) * norm_w (the next sub-layer's input norm).  Rows of N floats.
+// RMSNorm(x[m, :]) * norm_w (the next sub-layer's input norm) in out_form
+// (LX_ACT_*).  splits 0: x is left alone, the norm only.  Rows of N floats.
 int splitk_resid_rmsnorm(const float* ws, int splits, int M, int N, const float* bias, float* x,
                          const float* norm_w, float eps, float* hn, hipStream_t stream,
-                         int out_packed = 0);
+                         int out_form = 0);
 // v = sum_s ws[s][m, :] + bias over the fused q|k|v row (n_heads + 2 n_kv_heads
 // heads of 64); NEOX rotary at position pos[m] on the q and k heads; q ->
 // q_out[m, 0:n_heads*64] (row stride ldq), k / v -> k_cache / v_cache row
@@ -131,12 +140,12 @@ int splitk_qkv_rope_cache(const float* ws, int splits, int M, const float* bias,
                           int n_kv_heads, const int* pos, const float* inv_freq, float* q_out,
                           int ldq, float* k_cache, float* v_cache, int row0, hipStream_t stream);
 
-// lx_adaln_resid_f32, with y as two-part packed rows when out_packed
-// (lx_adaln_resid_packed_f32).
+// lx_adaln_resid_f32, with y in out_form (LX_ACT_*; LX_ACT_PACKED:
+// lx_adaln_resid_packed_f32).
 int adaln_resid(float* h, const float* partials, int splits, long partial_stride,
                 const float* bias, const float* gate, long gate_stride, const float* shift,
                 const float* scale, long mod_stride, float* y, int B, int T, int D, float eps,
-                int out_packed, hipStream_t stream);
+                int out_form, hipStream_t stream);
 
 // ---- split-operand GEMM with W in fragment order (lx_gemm_bx.hip) ----
 // lx_linear_bx_f32 (arguments and outputs as declared in lx_ops.h).
@@ -145,11 +154,37 @@ int linear_bx(const lx_linear_bx& g, hipStream_t stream);
 // bm-row tiles (0: the split tail does not apply), and the ws it needs.
 int bx_split_parts(int M, int N, int K, int bm);
 size_t bx_split_ws_floats(int bm);
+// ---- split-operand GEMM for few rows (lx_gemm_fs.hip) ----
+// y = epi(A W^T + bias), A in fragment order (a_frag: LX_ACT_FRAG2 / FRAG3 rows by
+// the product count) or fp32 rows (lda), W = wfrag_pack.  out: FS_OUT_F32 rows,
+// FS_OUT_PACKED two-part packed rows from column pack_from, FS_OUT_FRAG the
+// next projection's fragment-order A (GELU, SWIGLU_PAIRED), FS_OUT_PARTIAL raw
+// products of `slices` K slices.
+enum { FS_OUT_F32 = 0, FS_OUT_PARTIAL = 1, FS_OUT_PACKED = 2, FS_OUT_FRAG = 3 };
+struct FsLinear {
+  const void* A = nullptr;
+  long lda = 0;
+  int a_frag = 1;
+  const void* Wf = nullptr;
+  const float* bias = nullptr;
+  const lx_epilogue* epi = nullptr;
+  int out = FS_OUT_F32;
+  float* Y = nullptr;
+  long ldy = 0, slice_stride = 0;
+  int M = 0, N = 0, K = 0, slices = 1, products = 3, pack_from = 0;
+  // q|k|v projection of the LM: bias, NEOX rotary at pos[m] on the first
+  // rope_heads heads of 64, q -> Y, k / v -> the caches' row m (kv_cols wide)
+  const int* neox_pos = nullptr;
+  int q_cols = 0, kv_cols = 0, rope_heads = 0;
+  const float* rope_cs = nullptr;  // rope_table of the positions
+  float *k_cache = nullptr, *v_cache = nullptr;
+};
+int linear_fs(const FsLinear& g, hipStream_t stream);
 // lx_attention_f32 with the split-operand kernel's product count (3 or 6; the
-// fp32 kernel, which small grids run, ignores it).
+// fp32 kernel, which small grids run, ignores it); o in out_form (LX_ACT_*).
 int attention(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, float* o,
               int ldo, int B, int Tq, int Tk, int n_heads, int n_kv_heads, int head_dim,
-              float scale, int causal, int q_offset, int products, int out_packed,
+              float scale, int causal, int q_offset, int products, int out_form,
               hipStream_t stream, int kv_packed = 0);
 // Whether attention() runs this shape on the three-product split kernel, the
 // one that reads K and V as two-part packed rows (kv_packed).

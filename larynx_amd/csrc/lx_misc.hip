@@ -199,6 +199,22 @@ int fill_batch(float* dst, const float* src, long n, int copies, int zero_tail,
   return check_launch("fill_batch_kernel");
 }
 
+__global__ void rope_table_kernel(const float* __restrict__ inv_freq, float* tab, int n) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n * 32) return;
+  const int p = t >> 5, i = t & 31;
+  float s, c;
+  sincosf((float)p * inv_freq[i], &s, &c);
+  tab[p * 64 + i] = c;
+  tab[p * 64 + 32 + i] = s;
+}
+
+int rope_table(const float* inv_freq, int n, float* tab, hipStream_t stream) {
+  hipLaunchKernelGGL(rope_table_kernel, dim3((n * 32 + 255) / 256), dim3(256), 0, stream, inv_freq,
+                     tab, n);
+  return check_launch("rope_table_kernel");
+}
+
 int iota_i32(int* p, int n, hipStream_t stream) {
   hipLaunchKernelGGL(iota_kernel, dim3(grid1d(n)), dim3(256), 0, stream, p, n);
   return check_launch("iota_kernel");

@@ -34,7 +34,12 @@ struct Layer {
   void *qkv_wf = nullptr, *o_wf = nullptr, *gu_wf = nullptr, *down_wf = nullptr;
 };
 
-// K slices of a prefill projection on the fragment-order GEMM (64-row tiles):
+// Six products run on the fragment-operand GEMMs up to this many rows (64 rows 1.05x
+// the split-operand GEMM's prefill; 100 rows 0.93x: three parts per operand make
+// their tiles wait on the L2s).
+constexpr int kFragRows6 = 64;
+
+// K slices of a prefill projection on the split-operand GEMM (64-row tiles):
 // as many as the reduce passes take (9) while tiles x slices stay within one
 // workgroup per CU, then the fewest that keep the same longest slice (slices
 // of ceil(steps / slices) 64-wide steps).  L = 256: q|k|v 7 slices of 2 steps
@@ -46,6 +51,18 @@ int prefill_bx_slices(int rows, int N, int K) {
   int most = (int)std::min<long>(std::min(9, steps), std::max<long>(1, 256 / tiles));
   const int per = (steps + most - 1) / most;
   return (steps + per - 1) / per;
+}
+
+// K slices of the prefill's down_proj on the fragment-operand GEMMs (the one
+// projection whose tiles leave K long), at most 8 and each at least 512 deep: up to 64
+// rows about one 32 x 32 tile per CU (L = 37: 4 slices 10.8 us, 8 12.1), else about one
+// 128 x 128 tile per CU (L = 256: 8 slices 13.0 us, 4 19.9; L = 1024: 4 30.9, 8 34.4;
+// L = 1531: 3 42.4, 2 47.8, and one slice on 64 x 128 tiles before 63.7).
+int prefill_down_slices(int rows, int N, int K) {
+  const int most = std::max(1, std::min(8, K / 512));
+  const long fine = (long)((rows + 31) / 32) * (N / 32);
+  const long wide = (long)((rows + 127) / 128) * (N / 128);
+  return (int)std::max<long>(1, std::min<long>(most, 256 / (rows <= 64 ? fine : wide)));
 }
 
 }  // namespace
@@ -76,6 +93,7 @@ struct lx_qwen2 {
   long part_stride = 0;       // floats per kv head in `part`
   int max_splits = 0;
   float* rope_tab = nullptr;  // device copy of the rotary inverse frequencies
+  float* rope_cs = nullptr;   // their cosines and sines at every position (rope_table)
   bool use_graph = true;      // replay the layer stack as one HIP graph
   hipStream_t cap_stream = nullptr;
   // [0]: the cache fits one attention split; [1 + c]: split class c
@@ -109,26 +127,25 @@ int lx::qwen2_own_tables(lx_qwen2* m) {
 namespace {
 
 // Width of the split-K partial workspace: the largest splits * rows * N over
-// the three split projections, and the gate/up launch's split-tail partials,
-// at every prefill length up to max_ctx; *tails = the most tail tiles.
+// the projections that run as K slices, and the gate/up launch's split-tail
+// partials, at every prefill length up to max_ctx; *tails = the most tail tiles.
 size_t splitk_ws_floats(int max_ctx, int H, int QKV, int I, int* tails) {
   size_t best = 0;
   *tails = 0;
-  // splits depend on M only through the tile count, so the largest M of each
-  // 64-row band (and max_ctx itself) bounds every length
-  for (int M = 64;; M += 64) {
+  // splits depend on M only through its 32-row block count, so the largest M of
+  // each band (and max_ctx itself) bounds every length
+  for (int M = 32;; M += 32) {
     const int rows = M < max_ctx ? M : max_ctx;
     const int shapes[3][2] = {{QKV, H}, {H, H}, {H, I}};
     for (const auto& sh : shapes) {
       int ks = 0;
       const int splits = gemm_splitk_plan(rows, sh[0], sh[1], &ks);
       const int bx = prefill_bx_slices(rows, sh[0], sh[1]);
-      const size_t n = (size_t)std::max(splits, bx) * rows * sh[0];
-      if (n > best) best = n;
+      best = std::max(best, (size_t)std::max(splits, bx) * rows * sh[0]);
     }
+    best = std::max(best, (size_t)prefill_down_slices(rows, H, I) * rows * H);
     int t = 0;
-    const size_t nt = split_tail_ws_floats(rows, 2 * I, H, &t);
-    if (nt > best) best = nt;
+    best = std::max(best, split_tail_ws_floats(rows, 2 * I, H, &t));
     if (t > *tails) *tails = t;
     if (M >= max_ctx) break;
   }
@@ -138,7 +155,7 @@ size_t splitk_ws_floats(int max_ctx, int H, int QKV, int I, int* tails) {
 // q|k|v, o_proj or down_proj as K-slice partial products into m->ws; returns the
 // slice count through *splits.
 int prefill_partials(lx_qwen2* m, const float* x, int ldx, const void* wf, const float* w,
-                     int rows, int N, int K, int* splits, hipStream_t s, bool x_packed = false) {
+                     int rows, int N, int K, int* splits, hipStream_t s) {
   if (m->frag) {
     const int sl = prefill_bx_slices(rows, N, K);
     lx_linear_bx g{};
@@ -155,7 +172,6 @@ int prefill_partials(lx_qwen2* m, const float* x, int ldx, const void* wf, const
     g.bm = 64;
     g.slices = sl;
     g.products = m->products;
-    g.a_packed = x_packed ? 1 : 0;
     *splits = sl;
     return linear_bx(g, s);
   }
@@ -167,33 +183,96 @@ int prefill_partials(lx_qwen2* m, const float* x, int ldx, const void* wf, const
 // Prefill layer (src/llm/llm.cpp:141-173) over L rows at positions m->pos[0..L).
 // On entry m->hn holds input_layernorm(x); on exit x is the layer output and
 // m->hn holds next_norm(x) (the next layer's input_layernorm or the final norm).
-//   q/k/v: K-slice partials, then bias + NEOX rotary + cache append in one pass;
+// With fragment-order weights (m->frag: N multiples of 128, K of 64):
+//   q|k|v with bias, NEOX rotary and the cache append in its epilogue;
 //   attention (causal, GQA) reads q and the cache;
-//   o_proj: K-slice partials, then residual + post_attention_layernorm;
+//   o_proj adds to x in its epilogue; post_attention_layernorm;
 //   gate/up with the SwiGLU epilogue;
-//   down_proj: K-slice partials, then residual + next_norm.
-// Every projection runs on the fragment-order split-operand GEMM when the
-// geometry allows (m->frag: N multiples of 128, K of 64), else on the fp32 GEMMs.
-// With three products on the fragment-order GEMM, the GEMM inputs written by
-// this layer's kernels (attention's output, the RMSNorm outputs) are two-part
-// packed rows (bit-identical products, no split per column tile); hn_packed:
-// m->hn arrives packed (written by the previous layer), pack_next: write the
-// next norm packed (not the final norm, which the fp32 logits GEMM reads).
-int prefill_layer(lx_qwen2* m, Layer& L, int rows, const float* next_norm, hipStream_t s,
-                  bool hn_packed, bool pack_next) {
+//   down_proj: K-slice partials, then residual + next_norm in one pass.
+// Every GEMM input (the RMSNorms' and attention's output, SwiGLU's) is written in
+// fragment order by its producer; the last norm is fp32 (the logits GEMM reads it).
+int prefill_layer_frag(lx_qwen2* m, Layer& L, int rows, const float* next_norm, hipStream_t s,
+                       bool last) {
   const int H = m->H, KV = m->KV, QKV = m->QKV;
-  const bool pk = m->frag && m->products == 3;
+  const int form = m->products == 3 ? LX_ACT_FRAG2 : LX_ACT_FRAG3;
+  FsLinear g;
+  g.M = rows;
+  g.products = m->products;
+  FsLinear q = g;
+  q.A = m->hn;
+  q.Wf = L.qkv_wf;
+  q.bias = L.qkv_b;
+  q.Y = m->qkv;
+  q.ldy = QKV;
+  q.N = QKV;
+  q.K = H;
+  q.neox_pos = m->pos;
+  q.q_cols = H;
+  q.kv_cols = KV;
+  q.rope_heads = m->NH + m->NKV;
+  q.rope_cs = m->rope_cs;
+  q.k_cache = L.k_cache;
+  q.v_cache = L.v_cache;
+  LX_TRY(linear_fs(q, s));
+  const float scale = 1.0f / std::sqrt((float)m->HD);
+  LX_TRY(attention(m->qkv, QKV, L.k_cache, KV, L.v_cache, KV, m->att, H, 1, rows, rows, m->NH,
+                   m->NKV, m->HD, scale, /*causal*/ 1, /*q_offset*/ 0, /*products*/ 6, form, s));
+  lx_epilogue resid{};
+  resid.kind = LX_EPI_RESID;
+  FsLinear o = g;
+  o.A = m->att;
+  o.Wf = L.o_wf;
+  o.epi = &resid;
+  o.Y = m->x;
+  o.ldy = H;
+  o.N = H;
+  o.K = H;
+  LX_TRY(linear_fs(o, s));
+  LX_TRY(splitk_resid_rmsnorm(nullptr, 0, rows, H, nullptr, m->x, L.post_norm, m->eps, m->hn, s,
+                              form));
+  lx_epilogue swiglu{};
+  swiglu.kind = LX_EPI_SWIGLU_PAIRED;
+  FsLinear gu = g;
+  gu.A = m->hn;
+  gu.Wf = L.gu_wf;
+  gu.epi = &swiglu;
+  gu.out = FS_OUT_FRAG;
+  gu.Y = m->act;
+  gu.ldy = m->I;
+  gu.N = 2 * m->I;
+  gu.K = H;
+  LX_TRY(linear_fs(gu, s));
+  FsLinear d = g;
+  d.A = m->act;
+  d.Wf = L.down_wf;
+  d.out = FS_OUT_PARTIAL;
+  d.Y = m->ws;
+  d.ldy = H;
+  d.slice_stride = (long)rows * H;
+  d.N = H;
+  d.K = m->I;
+  d.slices = prefill_down_slices(rows, H, m->I);
+  LX_TRY(linear_fs(d, s));
+  return splitk_resid_rmsnorm(m->ws, d.slices, rows, H, nullptr, m->x, next_norm, m->eps, m->hn, s,
+                              last ? LX_ACT_F32 : form);
+}
+
+// The same layer with fp32 activations: six products past kFragRows6 rows, and
+// geometries the fragment tiles do not cover (on the fp32 GEMMs).  q|k|v, o_proj
+// and down_proj run as K-slice partials whose reduce passes apply bias + rotary +
+// cache append, or residual + the next norm.
+int prefill_layer(lx_qwen2* m, Layer& L, int rows, const float* next_norm, hipStream_t s) {
+  const int H = m->H, KV = m->KV, QKV = m->QKV;
   int sp = 0;
-  LX_TRY(prefill_partials(m, m->hn, H, L.qkv_wf, L.qkv_w, rows, QKV, H, &sp, s, pk && hn_packed));
+  LX_TRY(prefill_partials(m, m->hn, H, L.qkv_wf, L.qkv_w, rows, QKV, H, &sp, s));
   LX_TRY(splitk_qkv_rope_cache(m->ws, sp, rows, L.qkv_b, m->NH, m->NKV, m->pos, m->rope_tab,
                                m->qkv, QKV, L.k_cache, L.v_cache, 0, s));
   const float scale = 1.0f / std::sqrt((float)m->HD);
   LX_TRY(attention(m->qkv, QKV, L.k_cache, KV, L.v_cache, KV, m->att, H, 1, rows, rows, m->NH,
                    m->NKV, m->HD, scale, /*causal*/ 1, /*q_offset*/ 0, /*products*/ 6,
-                   /*out_packed*/ pk ? 1 : 0, s));
-  LX_TRY(prefill_partials(m, m->att, H, L.o_wf, L.o_w, rows, H, H, &sp, s, pk));
-  LX_TRY(splitk_resid_rmsnorm(m->ws, sp, rows, H, nullptr, m->x, L.post_norm, m->eps, m->hn, s,
-                              pk));
+                   LX_ACT_F32, s));
+  LX_TRY(prefill_partials(m, m->att, H, L.o_wf, L.o_w, rows, H, H, &sp, s));
+  LX_TRY(splitk_resid_rmsnorm(m->ws, sp, rows, H, nullptr, m->x, L.post_norm, m->eps, m->hn, s));
   lx_epilogue swiglu{};
   swiglu.kind = LX_EPI_SWIGLU_PAIRED;
   if (m->frag) {
@@ -211,7 +290,6 @@ int prefill_layer(lx_qwen2* m, Layer& L, int rows, const float* next_norm, hipSt
       g.n_counters = m->n_arrivals;
     }
     g.A = m->hn;
-    g.a_packed = pk ? 1 : 0;
     g.lda = H;
     g.Wf = L.gu_wf;
     g.epi = &swiglu;
@@ -230,8 +308,7 @@ int prefill_layer(lx_qwen2* m, Layer& L, int rows, const float* next_norm, hipSt
                              &swiglu, m->ws, m->ws_floats, m->arrivals, m->n_arrivals, s));
   }
   LX_TRY(prefill_partials(m, m->act, m->I, L.down_wf, L.down_w, rows, H, m->I, &sp, s));
-  return splitk_resid_rmsnorm(m->ws, sp, rows, H, nullptr, m->x, next_norm, m->eps, m->hn, s,
-                              pk && pack_next);
+  return splitk_resid_rmsnorm(m->ws, sp, rows, H, nullptr, m->x, next_norm, m->eps, m->hn, s);
 }
 
 // One decode layer (src/llm/llm.cpp:254-289): RMSNorm + QKV + rotary + cache
@@ -389,7 +466,7 @@ extern "C" int lx_qwen2_create(const lx_qwen2_weights* w, int max_ctx, lx_qwen2*
   // the fragment-order GEMM needs N multiples of 128 and K of 64 in every
   // prefill projection, and each activation below 2 GiB
   m->frag = QKV % 128 == 0 && H % 128 == 0 && (2 * I) % 128 == 0 && I % 64 == 0 &&
-            (size_t)max_ctx * I * 4 < (1ull << 31);
+            act_floats(max_ctx, I) * sizeof(float) < (1ull << 31);
   Arena& a = m->arena;
   bool ok = true;
   auto A = [&](size_t n) {
@@ -420,10 +497,10 @@ extern "C" int lx_qwen2_create(const lx_qwen2_weights* w, int max_ctx, lx_qwen2*
   }
   const size_t rows = max_ctx;
   m->x = A(rows * H);
-  m->hn = A(rows * H);
+  m->hn = A(act_floats(rows, H));
   m->qkv = A(rows * QKV);
-  m->att = A(rows * H);
-  m->act = A(rows * I);
+  m->att = A(act_floats(rows, H));
+  m->act = A(act_floats(rows, I));
   int tails = 0;
   m->ws_floats = std::max(splitk_ws_floats(max_ctx, H, QKV, I, &tails), bx_split_ws_floats(64));
   m->ws = A(m->ws_floats);
@@ -438,6 +515,7 @@ extern "C" int lx_qwen2_create(const lx_qwen2_weights* w, int max_ctx, lx_qwen2*
   m->pos = a.alloc<int>(max_ctx);
   m->d_pos = a.alloc<int>(1);
   m->rope_tab = A(m->HD / 2);
+  m->rope_cs = m->frag ? A((size_t)max_ctx * m->HD) : nullptr;
   ok = ok && m->pos && m->d_pos;
   if (!ok) {
     delete m;
@@ -501,6 +579,7 @@ extern "C" int lx_qwen2_create(const lx_qwen2_weights* w, int max_ctx, lx_qwen2*
     set_error("qwen2_create: rotary table upload failed");
     rc = LX_ERR_LAUNCH;
   }
+  if (rc == LX_OK && m->rope_cs) rc = rope_table(m->rope_tab, max_ctx, m->rope_cs, s);
   if (rc == LX_OK && hipStreamSynchronize(s) != hipSuccess) {
     set_error("qwen2_create: weight packing failed");
     rc = LX_ERR_LAUNCH;
@@ -568,11 +647,16 @@ extern "C" int lx_qwen2_prefill(lx_qwen2* m, const float* lm_input, int L, float
     return LX_ERR_LAUNCH;
   }
   m->cache_len = 0;
-  LX_TRY(lx_rmsnorm_f32(m->x, m->layers[0].in_norm, m->hn, L, H, m->eps, s));
+  const bool frag = m->frag && (m->products == 3 || L <= kFragRows6);
+  if (frag)
+    LX_TRY(splitk_resid_rmsnorm(nullptr, 0, L, H, nullptr, m->x, m->layers[0].in_norm, m->eps,
+                                m->hn, s, m->products == 3 ? LX_ACT_FRAG2 : LX_ACT_FRAG3));
+  else
+    LX_TRY(lx_rmsnorm_f32(m->x, m->layers[0].in_norm, m->hn, L, H, m->eps, s));
   for (int l = 0; l < m->NL; ++l) {
     const float* next_norm = l + 1 < m->NL ? m->layers[l + 1].in_norm : m->final_norm;
-    LX_TRY(prefill_layer(m, m->layers[l], L, next_norm, s, /*hn_packed*/ l > 0,
-                         /*pack_next*/ l + 1 < m->NL));
+    LX_TRY(frag ? prefill_layer_frag(m, m->layers[l], L, next_norm, s, l + 1 == m->NL)
+                : prefill_layer(m, m->layers[l], L, next_norm, s));
     if (hidden)
       (void)hipMemcpyAsync(hidden + (size_t)l * L * H, m->x, sizeof(float) * (size_t)L * H,
                            hipMemcpyDeviceToDevice, s);

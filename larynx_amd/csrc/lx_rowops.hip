@@ -118,12 +118,12 @@ __global__ __launch_bounds__(kRowsPerBlock * kWave) void adaln_kernel(
 // projection epilogue's own expression (h + (acc + bias) * gate).  The
 // (1 + scale), shift and gate rows of the batches a block touches and the bias
 // are staged in LDS.
-template <int NV, int SMAX>
+template <int NV, int SMAX, bool FRAG = false>
 __global__ __launch_bounds__(kRowsPerBlock * kWave) void adaln_resid_kernel(
     float* h, const float* P, int S, long pstride, const float* __restrict__ bias,
     const float* __restrict__ gate, long gate_stride, const float* __restrict__ shift,
     const float* __restrict__ scale, long mod_stride, float* y, int rows, int T, int D,
-    float eps, int pk, int gpb) {
+    float eps, int form, int gpb) {
   extern __shared__ float smem[];
   const int D4 = D >> 2;
   const int row0 = blockIdx.x * gpb * kRowsPerBlock;
@@ -234,7 +234,6 @@ __global__ __launch_bounds__(kRowsPerBlock * kWave) void adaln_resid_kernel(
       const float rstd = 1.0f / sqrtf(var + eps);
       const float4* s1 = reinterpret_cast<const float4*>(smem + (3 * bi) * D);
       const float4* s2 = reinterpret_cast<const float4*>(smem + (3 * bi + 1) * D);
-      float4* yr = reinterpret_cast<float4*>(y + (long)row * D);
 #pragma unroll
       for (int j = 0; j < NV; ++j) {
         const int i = lane + j * kWave;
@@ -245,10 +244,13 @@ __global__ __launch_bounds__(kRowsPerBlock * kWave) void adaln_resid_kernel(
           o.y = ((v[j].y - mean) * rstd) * m.y + sh.y;
           o.z = ((v[j].z - mean) * rstd) * m.z + sh.z;
           o.w = ((v[j].w - mean) * rstd) * m.w + sh.w;
-          if (pk)  // two-part packed row for the three-product GEMM
-            reinterpret_cast<uintx4_t*>(yr)[i] = pack2_bf16(floatx4{o.x, o.y, o.z, o.w});
+          if (FRAG)
+            act_store4(y, D, row, 4 * i, floatx4{o.x, o.y, o.z, o.w}, form);
+          else if (form)  // two-part packed row for the three-product GEMM
+            reinterpret_cast<uintx4_t*>(y + (long)row * D)[i] =
+                pack2_bf16(floatx4{o.x, o.y, o.z, o.w});
           else
-            yr[i] = o;
+            reinterpret_cast<float4*>(y + (long)row * D)[i] = o;
         }
       }
     }
@@ -351,7 +353,7 @@ namespace lx {
 int adaln_resid(float* h, const float* partials, int splits, long partial_stride,
                 const float* bias, const float* gate, long gate_stride, const float* shift,
                 const float* scale, long mod_stride, float* y, int B, int T, int D, float eps,
-                int out_packed, hipStream_t stream) {
+                int out_form, hipStream_t stream) {
   LX_REQUIRE(h && shift && scale, "adaln_resid: null pointer");
   LX_REQUIRE(B > 0 && T > 0 && D > 0, "adaln_resid: bad shape B=%d T=%d D=%d", B, T, D);
   LX_REQUIRE(D % 4 == 0 && D <= 16 * 256, "adaln_resid: D=%d must be a multiple of 4, <= 4096",
@@ -362,6 +364,8 @@ int adaln_resid(float* h, const float* partials, int splits, long partial_stride
                              gate_stride % 4 == 0),
              "adaln_resid: bad partials / gate");
   LX_REQUIRE(splits > 0 || y, "adaln_resid: nothing to do");
+  LX_REQUIRE(out_form < LX_ACT_FRAG2 || (D % 16 == 0 && splits == 0),
+             "adaln_resid: fragment order needs D %% 16 and no partials");
   LX_REQUIRE((mod_stride == 0 || mod_stride >= D) && mod_stride % 4 == 0,
              "adaln_resid: bad mod_stride %ld", mod_stride);
   LX_REQUIRE(((uintptr_t)h | (uintptr_t)y | (uintptr_t)shift | (uintptr_t)scale |
@@ -381,11 +385,17 @@ int adaln_resid(float* h, const float* partials, int splits, long partial_stride
   const int nblk = (rows + rpb - 1) / rpb;
   LX_REQUIRE(splits == 0 || D <= 8 * 256, "adaln_resid: D=%d above 2048 with partials", D);
   const int nv = (D / 4 + kWave - 1) / kWave;
-#define LX_AR(NVV, SM)                                                                          \
-  hipLaunchKernelGGL((adaln_resid_kernel<NVV, SM>), dim3(nblk), dim3(kRowsPerBlock * kWave), lds,     \
+#define LX_AR(NVV, SM, ...)                                                                     \
+  hipLaunchKernelGGL((adaln_resid_kernel<NVV, SM, ##__VA_ARGS__>), dim3(nblk), dim3(kRowsPerBlock * kWave), lds,     \
                      stream, h, partials, splits, partial_stride, bias, gate, gate_stride, shift, \
-                     scale, mod_stride, y, rows, T, D, eps, out_packed ? 1 : 0, gpb)
-  if (nv <= 4 && splits <= 2)
+                     scale, mod_stride, y, rows, T, D, eps, out_form, gpb)
+  if (out_form >= LX_ACT_FRAG2 && nv <= 4)
+    LX_AR(4, 0, true);
+  else if (out_form >= LX_ACT_FRAG2 && nv <= 8)
+    LX_AR(8, 0, true);
+  else if (out_form >= LX_ACT_FRAG2)
+    LX_AR(16, 0, true);
+  else if (nv <= 4 && splits <= 2)
     LX_AR(4, 2);
   else if (nv <= 4)
     LX_AR(4, 4);

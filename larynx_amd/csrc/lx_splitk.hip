@@ -52,7 +52,7 @@ __global__ __launch_bounds__(256) void resid_rmsnorm_kernel(const float* __restr
                                                             int splits, int M, int N,
                                                             const float* __restrict__ bias,
                                                             float* x, const float* __restrict__ w,
-                                                            float eps, float* hn, int pk) {
+                                                            float eps, float* hn, int form) {
   __shared__ float red[4];
   const int row = blockIdx.x, t = threadIdx.x;
   const int N4 = N >> 2;
@@ -62,6 +62,10 @@ __global__ __launch_bounds__(256) void resid_rmsnorm_kernel(const float* __restr
   for (int j = 0; j < NV; ++j) {
     const int i = min(t + 256 * j, N4 - 1);
     float4 a = xr[i];
+    if (splits == 0) {  // x is up to date: the norm alone
+      v[j] = t + 256 * j < N4 ? a : make_float4(0.f, 0.f, 0.f, 0.f);
+      continue;
+    }
     float4 sum = sum_slices(ws, splits, (long)M * N, (long)row * N, i);
     if (bias) {
       const float4 b = reinterpret_cast<const float4*>(bias)[i];
@@ -76,9 +80,10 @@ __global__ __launch_bounds__(256) void resid_rmsnorm_kernel(const float* __restr
     a.w = a.w + sum.w;
     v[j] = t + 256 * j < N4 ? a : make_float4(0.f, 0.f, 0.f, 0.f);
   }
+  if (splits > 0)
 #pragma unroll
-  for (int j = 0; j < NV; ++j)
-    if (t + 256 * j < N4) xr[t + 256 * j] = v[j];
+    for (int j = 0; j < NV; ++j)
+      if (t + 256 * j < N4) xr[t + 256 * j] = v[j];
   if (!w) return;
   // RMSNorm of the updated row
   float ss = 0.0f;
@@ -86,7 +91,6 @@ __global__ __launch_bounds__(256) void resid_rmsnorm_kernel(const float* __restr
   for (int j = 0; j < NV; ++j)
     ss += (v[j].x * v[j].x + v[j].y * v[j].y) + (v[j].z * v[j].z + v[j].w * v[j].w);
   const float r = 1.0f / sqrtf(block_sum256(ss, red) / (float)N + eps);
-  float4* hr = reinterpret_cast<float4*>(hn + (long)row * N);
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int i = t + 256 * j;
@@ -97,10 +101,7 @@ __global__ __launch_bounds__(256) void resid_rmsnorm_kernel(const float* __restr
       o.y = (v[j].y * r) * g.y;
       o.z = (v[j].z * r) * g.z;
       o.w = (v[j].w * r) * g.w;
-      if (pk)  // two-part packed row for the three-product GEMM
-        reinterpret_cast<uintx4_t*>(hr)[i] = pack2_bf16(floatx4{o.x, o.y, o.z, o.w});
-      else
-        hr[i] = o;
+      act_store4(hn, N, row, 4 * i, floatx4{o.x, o.y, o.z, o.w}, form);
     }
   }
 }
@@ -160,20 +161,21 @@ __global__ __launch_bounds__(256) void qkv_rope_cache_kernel(
 
 int splitk_resid_rmsnorm(const float* ws, int splits, int M, int N, const float* bias, float* x,
                          const float* norm_w, float eps, float* hn, hipStream_t stream,
-                         int out_packed) {
-  LX_REQUIRE(ws && x && M > 0 && N > 0 && N % 4 == 0 && splits >= 1 && splits <= kMaxSplits &&
-                 (!norm_w || hn),
+                         int out_form) {
+  LX_REQUIRE((ws || splits == 0) && x && M > 0 && N > 0 && N % 4 == 0 && splits >= 0 &&
+                 splits <= kMaxSplits && (norm_w ? hn != nullptr : splits > 0) &&
+                 (out_form < LX_ACT_FRAG2 || N % 16 == 0),
              "splitk_resid_rmsnorm: bad args");
   const int nv = (N / 4 + 255) / 256;
   if (nv <= 1)
     hipLaunchKernelGGL(resid_rmsnorm_kernel<1>, dim3(M), dim3(256), 0, stream, ws, splits, M, N,
-                       bias, x, norm_w, eps, hn, out_packed ? 1 : 0);
+                       bias, x, norm_w, eps, hn, out_form);
   else if (nv <= 2)
     hipLaunchKernelGGL(resid_rmsnorm_kernel<2>, dim3(M), dim3(256), 0, stream, ws, splits, M, N,
-                       bias, x, norm_w, eps, hn, out_packed ? 1 : 0);
+                       bias, x, norm_w, eps, hn, out_form);
   else if (nv <= 4)
     hipLaunchKernelGGL(resid_rmsnorm_kernel<4>, dim3(M), dim3(256), 0, stream, ws, splits, M, N,
-                       bias, x, norm_w, eps, hn, out_packed ? 1 : 0);
+                       bias, x, norm_w, eps, hn, out_form);
   else {
     set_error("splitk_resid_rmsnorm: N=%d too wide", N);
     return LX_ERR_ARG;

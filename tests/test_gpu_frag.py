@@ -1,0 +1,73 @@
+"""The projections on fragment-order activations (lx_gemm_fs.hip, lx_gemm_ft.hip) through the
+estimator and the Qwen2 prefill, against the oracle at the row counts where a launch changes
+its tiles: part of one 32-row block, whole blocks and one row past them, the last row count of
+the 32 x 32 and 64 x 64 tiles, and the first past the fragment-order block."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import announce
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,T,products", [
+    (1, 5, 3), (2, 16, 3), (2, 17, 6), (2, 80, 3), (2, 83, 6), (1, 161, 3), (2, 160, 6),
+    (2, 161, 6), (2, 255, 3), (2, 257, 3),
+])
+def test_dit_projection_tiles_vs_oracle(gpu, B, T, products):
+    """Two blocks with O(1) modulation, so that every projection carries weight in the
+    result.  Tolerance: the two-part operands' 2^-16 per element, some ten roundings deep."""
+    from larynx_amd.flow import DiTConfig, DiTEstimator, dit_param_shapes
+    announce(f"dit B={B} T={T} products={products}")
+    cfg = DiTConfig(depth=2)
+    params = orc.make_params(dit_param_shapes(cfg), 29)
+    dparams = {k: torch.from_numpy(v).to(gpu) for k, v in params.items()}
+    est = DiTEstimator(dparams, cfg, B=B, max_T=max(T, 64))
+    est.set_products(products)
+    x, mu, cond = (orc.normal((B, 80, T), 31 + T, s) for s in (1, 2, 3))
+    spks = orc.normal((B, 80), 31, 4, 1.0 / np.sqrt(80.0))
+    t = np.linspace(0.2, 0.7, B).astype(np.float32)
+    dphi = est.forward(*(torch.from_numpy(a).to(gpu) for a in (x, mu, cond, spks, t)))
+    torch.cuda.synchronize()
+    est.close()
+    ref = orc.Dit(params, depth=2).forward(x, mu, cond, spks, t)
+    err = orc.rel_err(dphi.cpu().numpy(), ref)
+    assert err < (1e-4 if products == 3 else 2e-5), err
+
+
+@pytest.fixture(scope="module")
+def qwen2(gpu):
+    from larynx_amd.llm import Qwen2Config, Qwen2LM, qwen2_param_shapes
+    cfg = Qwen2Config(n_layers=2, text_vocab=2000)
+    params = orc.make_params(qwen2_param_shapes(cfg), 78)
+    for k in params:
+        if k.endswith("layernorm.weight") or k == "norm.weight":
+            params[k] = (params[k] + 1.0).astype(np.float32)
+    lm = Qwen2LM({k: torch.from_numpy(v).to(gpu) for k, v in params.items()}, cfg, max_ctx=1100)
+    yield cfg, params, lm
+    lm.close()
+
+
+@pytest.mark.parametrize("L,products", [
+    (1, 6), (31, 3), (32, 3), (33, 6), (65, 3), (129, 3), (129, 6), (545, 3), (1089, 3),
+])
+def test_prefill_projection_tiles_vs_oracle(gpu, qwen2, L, products):
+    """q|k|v with the rotary and cache append in its epilogue, o_proj's residual epilogue,
+    gate/up with SwiGLU in fragment order and down_proj's K slices."""
+    cfg, params, lm = qwen2
+    announce(f"qwen2 prefill L={L} products={products}")
+    lm.set_products(products)
+    lm_in = torch.from_numpy(orc.normal((L, cfg.hidden), 500 + L, 1, 0.5)).to(gpu)
+    logits, hidden, final = lm.prefill(lm_in, capture=True)
+    torch.cuda.synchronize()
+    o = orc.Qwen2(params, cfg, cap=1100)
+    rl, rh, rf = o.prefill(lm_in.cpu().numpy(), capture=True)
+    tol = 5e-5 if products == 3 else 1e-5
+    for layer in range(cfg.n_layers):
+        assert orc.rel_err(hidden[layer].cpu().numpy(), rh[layer]) < tol, layer
+        k, v = lm.cache_views(layer)
+        assert orc.rel_err(k[:L].cpu().numpy(), o.k_cache[layer, :L]) < tol, layer
+        assert orc.rel_err(v[:L].cpu().numpy(), o.v_cache[layer, :L]) < tol, layer
+    assert orc.rel_err(logits.cpu().numpy(), rl) < tol
