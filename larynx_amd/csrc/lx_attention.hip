@@ -45,6 +45,7 @@ constexpr size_t flash_lds() {
   return (size_t)2 * (DB ? 2 : 1) * 32 * KS * kLD * sizeof(float);
 }
 
+
 // Four output channels: fp32, or (opk) a two-part packed group for the
 // three-product GEMM that consumes the attention output.
 __device__ __forceinline__ void store_o4(float* p, floatx4 w, int opk) {
@@ -576,8 +577,13 @@ __device__ __forceinline__ int vt_pos(int k) {
 // V of tile t + 1 replaces V of tile t - 1, so one barrier per tile suffices.
 // KVP: K and V arrive as two-part packed rows (their producer split them
 // once; three products), so staging stores the parts without splitting.
-template <int QS, int KS, bool BUF, int NP, bool KVP = false>
-__global__ __launch_bounds__(64 * QS * KS) void attn_bx_kernel(
+// OCC = 2: at most 256 registers, so that two 64-query workgroups of three products
+// (72 KB of LDS each) share a CU; the compiler's own choice is above 256, one
+// workgroup per CU, which is a little faster for grids of at most one per CU (T = 500
+// 16.6 against 17.7 us with the spills) and a round longer past that (T = 777 40.0 ->
+// 30.1 us, T = 1500 100.5 -> 83.8, T = 2500 264 -> 207).
+template <int QS, int KS, bool BUF, int NP, bool KVP = false, int OCC = 1>
+__global__ __launch_bounds__(64 * QS * KS) __attribute__((amdgpu_waves_per_eu(OCC))) void attn_bx_kernel(
     const float* __restrict__ q, int ldq, const float* __restrict__ k, int ldk,
     const float* __restrict__ v, int ldv, float* __restrict__ o, int ldo, int Tq, int Tk,
     int n_heads, int rep, float qscale, int causal, int q_offset, int opk) {
@@ -600,12 +606,19 @@ __global__ __launch_bounds__(64 * QS * KS) void attn_bx_kernel(
   const int qs = wave % QS, ks = wave / QS;
   const int lane = tid & 63, r = lane & 31, h = lane >> 5;
   const int nq = (Tq + kQT - 1) / kQT;
-  int work;
-  {
+  int qtile, bh;
+  if (causal) {
+    // a query tile's work grows with its position: the longest are dealt first, so
+    // that the short ones fill the last round
+    const int nbh = gridDim.x / nq;
+    qtile = nq - 1 - (int)blockIdx.x / nbh;
+    bh = blockIdx.x % nbh;
+  } else {
     const int n = gridDim.x, x = blockIdx.x & 7, per = n >> 3, rem = n & 7;
-    work = x * per + min(x, rem) + (blockIdx.x >> 3);
+    const int work = x * per + min(x, rem) + (blockIdx.x >> 3);
+    qtile = work % nq;
+    bh = work / nq;
   }
-  const int qtile = work % nq, bh = work / nq;
   const int head = bh % n_heads, b = bh / n_heads, g = head / rep;
   const int qt0 = qtile * kQT;
   const int q0 = qt0 + qs * 32;
@@ -1039,20 +1052,31 @@ __global__ __launch_bounds__(64 * QS * KS) void attn_bx_kernel(
 }
 
 }  // namespace
+// Causal grids smaller than the CUs take the split-operand kernel from this many
+// 64-query workgroups on.
+constexpr long kCausalSplit = 176;
+
 // Layout of a launch: 0 small grids (32-query workgroups), 1 64-query, 2
-// 128-query; and whether the split-operand kernel runs it (see attention()).
-static int attention_layout(int B, int Tq, int n_heads, int products, bool* split) {
+// 128-query; *np: the split-operand kernel's product count, 0 the fp32 kernel (see
+// attention()).
+static int attention_layout(int B, int Tq, int n_heads, int products, int causal, int* np) {
+  const long wg32 = (long)((Tq + 31) / 32) * n_heads * B;
   const long wg64 = (long)((Tq + 63) / 64) * n_heads * B;
   const long wg128 = (long)((Tq + 127) / 128) * n_heads * B;
-  const int layout = wg64 < 256 ? 0 : (wg128 % 256 == 0 ? 2 : 1);  // small / 64-query / wide
-  *split = layout == 2 || (layout == 1 && (wg64 <= 256 || products == 3));
+  if (wg64 < 256) {
+    const bool small = causal ? wg64 < kCausalSplit : wg32 <= 256;
+    *np = small ? 0 : 6;
+    return small ? 0 : 1;
+  }
+  const int layout = wg128 % 256 == 0 ? 2 : 1;
+  *np = layout == 2 || wg64 == 256 || products == 3 ? products : causal ? 6 : 0;
   return layout;
 }
 
 bool attention_takes_packed_kv(int B, int Tq, int n_heads, int products) {
-  bool split = false;
-  attention_layout(B, Tq, n_heads, products, &split);
-  return split && products == 3;
+  int np = 0;
+  attention_layout(B, Tq, n_heads, products, 0, &np);
+  return np == 3;
 }
 
 int attention(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, float* o,
@@ -1083,49 +1107,48 @@ int attention(const float* q, int ldq, const float* k, int ldk, const float* v, 
   const long lim = 1L << 31;
   const bool buf = ((long)(Tk + 128) * ldk + kHD) * 4 < lim && ((long)(Tk + 128) * ldv + kHD) * 4 < lim;
   // Three layouts.  64-query workgroups (2 query sub-tiles x 2 key parts, 64-key
-  // tiles double buffered, 70 KB of LDS) whenever they cover the CUs (DiT at
-  // T = 500: 256 workgroups, 24.9 us; T = 3000: 1504).  A grid smaller than
-  // the device (the Qwen2 prefill at L = 256: 56 workgroups) takes 32-query
-  // workgroups of 4 key parts over single-buffered 128-key tiles instead:
-  // twice the workgroups, four waves each (13.9 -> 9.8 us).  At T = 500 that
-  // layout is slower (27.8 us: the 4-part merge and two barriers per tile
-  // cost more than the second resident workgroup per CU returns).
-  // The third, 128-query workgroups of 4 query sub-tiles x 2 key parts (512
-  // threads: every K/V tile feeds twice the queries), replaces the
-  // 64-query layout when its grid is a whole number of workgroups per CU (fp32
-  // kernel: T = 3000, 768 workgroups, 612 -> 571 us; T = 2000 283 -> 262; T = 1000
-  // 75.9 -> 73.8).  Grids that
-  // leave a partial round (T = 1500: 384 workgroups; 2500: 640) run slower
-  // than the 64-query layout and keep it.
-  bool split = false;
-  const int layout = attention_layout(B, Tq, n_heads, products, &split);
-  // The split-operand kernel (attn_bx_kernel) runs the 128-query layout and
-  // the 64-query layout when its grid fits the CUs in one round (T = 500: 23.6
-  // vs 26.2 us; T = 1000: 59.7 vs 81.2; T = 2000: 210 vs 275; T = 3000: 450
-  // vs 571).  With 108 KB of LDS it keeps one workgroup per CU, so a 64-query
-  // grid of several rounds (T = 1500: 181 vs 170 us) and the small grids stay
-  // on the fp32 kernel, whose 70 KB (or single-buffered) LDS lets two
-  // workgroups share a CU.
-  // With three products (two bf16 parts per operand) the split kernel's K/V
-  // planes take 72 KB (64-query layout), so two of its workgroups share a CU
-  // and it also runs the 64-query grids of several rounds (T = 1500: 157 ->
-  // 99 us; T = 2500: 416 -> 263 us against the fp32 kernel).
-  const bool np3 = products == 3;
+  // tiles double buffered) whenever they cover the CUs.  A smaller grid takes
+  // 32-query workgroups of 4 key parts over single-buffered 128-key tiles on the fp32
+  // matrix cores while they number at most one per CU (twice the workgroups, four
+  // waves each; at T = 500 the 4-part merge and two barriers per tile cost more than
+  // that returns).  128-query workgroups (512 threads: every K/V tile feeds twice the
+  // queries) replace the 64-query ones when they are a whole number per CU (T = 1000,
+  // 2000, 3000 at B = 2, H = 16; three products T = 3000 230 us); grids that leave a
+  // partial round are faster on 64 queries.
+  //
+  // The split-operand kernel runs with the caller's product count on the 128-query
+  // layout, on one round of 64-query workgroups, and with three products on any
+  // number of them.  With six (108 KB of LDS, one workgroup per CU) several rounds
+  // are faster on the fp32 kernel, two of whose workgroups share a CU, except causal
+  // ones: their tiles are dealt longest first, so the rounds overlap (kCausalSplit).
+  // A grid between the two small layouts (T = 300: 320 32-query workgroups, a second
+  // round of the fp32 kernel) takes six products, whose error is that of fp32.
+  int np = 0;
+  const int layout = attention_layout(B, Tq, n_heads, products, causal, &np);
   // K / V as packed rows: the three-product split kernel only.
-  LX_REQUIRE(!kv_packed || (split && np3),
+  LX_REQUIRE(!kv_packed || np == 3,
              "attention: packed K/V need the three-product split kernel (B=%d Tq=%d)", B, Tq);
+  const int qt = layout == 0 ? 32 : layout == 1 ? 64 : 128;
+  const long nwg64 = (long)((Tq + qt - 1) / qt) * n_heads * B;
+  const bool two = nwg64 > 256;  // three products, 64 queries: more than one per CU
   auto pick = [&]() {
-    if (split && np3 && kv_packed) {
+    if (np == 3 && kv_packed) {
       if (layout == 2)
         return buf ? attn_bx_kernel<4, 2, true, 3, true> : attn_bx_kernel<4, 2, false, 3, true>;
+      if (two)
+        return buf ? attn_bx_kernel<2, 2, true, 3, true, 2>
+                   : attn_bx_kernel<2, 2, false, 3, true, 2>;
       return buf ? attn_bx_kernel<2, 2, true, 3, true> : attn_bx_kernel<2, 2, false, 3, true>;
     }
-    if (split && np3) {
+    if (np == 3) {
       if (layout == 2)
         return buf ? attn_bx_kernel<4, 2, true, 3> : attn_bx_kernel<4, 2, false, 3>;
+      if (two)
+        return buf ? attn_bx_kernel<2, 2, true, 3, false, 2>
+                   : attn_bx_kernel<2, 2, false, 3, false, 2>;
       return buf ? attn_bx_kernel<2, 2, true, 3> : attn_bx_kernel<2, 2, false, 3>;
     }
-    if (split) {
+    if (np == 6) {
       if (layout == 2)
         return buf ? attn_bx_kernel<4, 2, true, 6> : attn_bx_kernel<4, 2, false, 6>;
       return buf ? attn_bx_kernel<2, 2, true, 6> : attn_bx_kernel<2, 2, false, 6>;
@@ -1135,15 +1158,16 @@ int attention(const float* q, int ldq, const float* k, int ldk, const float* v, 
     return buf ? attn_flash_kernel<2, 2, true, true> : attn_flash_kernel<2, 2, true, false>;
   };
   auto kern = pick();
-  const int qt = layout == 0 ? 32 : layout == 1 ? 64 : 128;
   const int threads = layout == 2 ? 512 : 256;
   const size_t lds =
-      split ? (np3 ? (layout == 2 ? bx_lds<4, 2, 3>() : bx_lds<2, 2, 3>())
-                   : (layout == 2 ? bx_lds<4, 2, 6>() : bx_lds<2, 2, 6>()))
-            : (layout == 0 ? flash_lds<1, 4, false>() : flash_lds<2, 2, true>());
-  const int variant = split ? 2 + (layout == 2) + 2 * np3 + 2 * (kv_packed != 0) : layout;
-  static LdsLimit once[8][2];  // [kernel variant][buf]
-  const int rc = raise_lds_limit((const void*)kern, lds, once[variant][buf], "attention");
+      np ? (np == 3 ? (layout == 2 ? bx_lds<4, 2, 3>() : bx_lds<2, 2, 3>())
+                    : (layout == 2 ? bx_lds<4, 2, 6>() : bx_lds<2, 2, 6>()))
+         : (layout == 0 ? flash_lds<1, 4, false>() : flash_lds<2, 2, true>());
+  const int variant =
+      np ? 2 + (layout == 2) + 2 * (np == 3) + 2 * (kv_packed != 0) : layout;
+  static LdsLimit once[8][2][2];  // [kernel variant][two per CU][buf]
+  const int rc =
+      raise_lds_limit((const void*)kern, lds, once[variant][np == 3 && two][buf], "attention");
   if (rc) return rc;
   const long nwg = (long)((Tq + qt - 1) / qt) * n_heads * B;
   LX_REQUIRE(nwg < (1L << 31), "attention: %ld workgroups exceed the grid limit", nwg);
