@@ -29,6 +29,7 @@
 
 #include "lx_common.hpp"
 #include "lx_gemm_common.hpp"
+#include "lx_gemm_frag.hpp"
 #include "lx_internal.hpp"
 
 namespace lx {
@@ -689,6 +690,10 @@ int linear_bx(const lx_linear_bx& g, hipStream_t stream) {
                "linear_bx: bad output");
     ep.vec = epi_vec_ok(ep, g.Y, (int)g.ldy, g.bias);
     LX_REQUIRE(ep.vec, "linear_bx: y, bias and gate must be 16-byte aligned");
+  }
+  if (g.out != BX_OUT_PARTIAL && slices == 1 && !(g.ws && g.counters)) {
+    int frc = LX_OK;
+    if (linear_fs_rows(g, ep, stream, &frc)) return frc;
   }
   BxArgs a;
   a.A = g.A;

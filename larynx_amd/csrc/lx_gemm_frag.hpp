@@ -31,6 +31,10 @@ constexpr int kEpiNeox = 100;  // internal epilogue beside LX_EPI_*
 // 25.5 / 31.3; M = 1000, N = 2048: 128 tiles 26.0 / 21.6).
 constexpr int kFtWideTiles = 150;
 
+// lx_linear_bx of few rows (fp32 or packed, fp32 or packed output, one slice, arguments
+// checked) on the few-row kernel; the choice depends on the shape alone, so fp32 and
+// packed operands give the same bits.  false: not taken.
+bool linear_fs_rows(const lx_linear_bx& g, const EpiArgs& ep, hipStream_t stream, int* rc);
 int linear_ft(FsArgs a, int out, const EpiArgs& ep, int products, hipStream_t s);
 
 __device__ __forceinline__ sbf16x8 frag_bf(uintx4_t v) { return __builtin_bit_cast(sbf16x8, v); }

@@ -23,6 +23,10 @@ namespace {
 
 constexpr unsigned kOob = 1u << 31;  // past every operand (all are below 2 GiB): loads give zero
 
+// A operand: fp32 rows (split in registers), fragment order, two-part packed rows
+// (three products).  The last two hold the same parts as the first splits into.
+enum { kARows = 0, kAFrag = 1, kAPacked = 2 };
+
 template <int RB, int CB, int NP>
 constexpr int fs_depth() {
   constexpr int NPL = NP == 6 ? 3 : 2;
@@ -52,7 +56,7 @@ __global__ __launch_bounds__(64 * KW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gemm_fs_kernel(FsArgs a, EpiArgs ep) {
   constexpr int NPL = NP == 6 ? 3 : 2;
   constexpr int D = fs_depth<RB, CB, NP>();
-  constexpr int AV = AF ? NPL : 2;  // 16-byte loads per A fragment set
+  constexpr int AV = AF == kAFrag ? NPL : 2;  // 16-byte loads per A fragment set
   extern __shared__ __attribute__((aligned(16))) float red[];  // [KW][RB * CB * 4][64] float4
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -81,7 +85,7 @@ gemm_fs_kernel(FsArgs a, EpiArgs ep) {
   const int nrb = (a.M + 31) / 32;
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
-    if (AF)
+    if (AF == kAFrag)
       oa[i] = rb0 + i < nrb ? (unsigned)(rb0 + i) * nks * (NPL * 1024) + lane * 16 : kOob;
     else
       oa[i] = (unsigned)min((rb0 + i) * 32 + r, a.M - 1) * (unsigned)(a.lda * 4) + h * 32;
@@ -92,7 +96,7 @@ gemm_fs_kernel(FsArgs a, EpiArgs ep) {
   uintx4_t fa[D][RB][AV], fw[D][CB][NPL];
   auto load = [&](int i, int s) {  // k step k0 + s into ring slot i; past the range: no access
     const unsigned past = s < n ? 0u : kOob;
-    const int sa = (k0 + s) * (AF ? NPL * 1024 : 64), sw = (k0 + s) * 3072;
+    const int sa = (k0 + s) * (AF == kAFrag ? NPL * 1024 : 64), sw = (k0 + s) * 3072;
 #pragma unroll
     for (int c = 0; c < CB; ++c)
 #pragma unroll
@@ -104,7 +108,7 @@ gemm_fs_kernel(FsArgs a, EpiArgs ep) {
 #pragma unroll
       for (int p = 0; p < AV; ++p)
         fa[i][b][p] = __builtin_amdgcn_raw_buffer_load_b128(
-            ars, (oa[b] + sa + p * (AF ? 1024 : 16)) | past, 0, 0);
+            ars, (oa[b] + sa + p * (AF == kAFrag ? 1024 : 16)) | past, 0, 0);
   };
   constexpr int kPa6[6] = {2, 1, 0, 1, 0, 0}, kPw6[6] = {0, 1, 2, 0, 1, 0};
   constexpr int kPa3[3] = {1, 0, 0}, kPw3[3] = {0, 1, 0};
@@ -137,9 +141,15 @@ gemm_fs_kernel(FsArgs a, EpiArgs ep) {
       uintx4_t f[RB][NPL];
 #pragma unroll
       for (int b = 0; b < RB; ++b) {
-        if (AF) {
+        if (AF == kAFrag) {
 #pragma unroll
           for (int p = 0; p < NPL; ++p) f[b][p] = fa[i][b][p];
+        } else if (AF == kAPacked) {
+#pragma unroll
+          for (int p = 0; p < NPL; ++p) {
+            const uintx4_t lo = fa[i][b][0], hi = fa[i][b][1];
+            f[b][p] = uintx4_t{lo[2 * p], lo[2 * p + 1], hi[2 * p], hi[2 * p + 1]};
+          }
         } else {
           fs_split<NPL>(fa[i][b][0], fa[i][b][1], f[b]);
         }
@@ -215,7 +225,7 @@ template <int RB, int CB, int KW, int NP, int AF>
 int dispatch_fs(FsArgs a, int out, const EpiArgs& ep, hipStream_t s) {
   a.tiles_m = (a.M + 32 * RB - 1) / (32 * RB);
   a.tiles_n = a.N / (32 * CB);
-  if constexpr (AF == 1) {
+  if constexpr (AF == kAFrag) {
     if (out == FS_OUT_PARTIAL)
       return launch_fs<LX_EPI_NONE, RB, CB, KW, FS_OUT_PARTIAL, NP, AF>(a, ep, s);
     if (out == FS_OUT_FRAG) {
@@ -226,6 +236,20 @@ int dispatch_fs(FsArgs a, int out, const EpiArgs& ep, hipStream_t s) {
     if constexpr (NP == 3)
       if (out == FS_OUT_PACKED)
         return launch_fs<LX_EPI_ROPE_PARTIAL, RB, CB, KW, FS_OUT_PACKED, NP, AF>(a, ep, s);
+  }
+  if constexpr (AF != kAFrag) {
+    if constexpr (NP == 3)
+      if (out == FS_OUT_PACKED) {
+        if (ep.kind == LX_EPI_ROPE_PARTIAL)
+          return launch_fs<LX_EPI_ROPE_PARTIAL, RB, CB, KW, FS_OUT_PACKED, NP, AF>(a, ep, s);
+        if (ep.kind == LX_EPI_GELU_TANH)
+          return launch_fs<LX_EPI_GELU_TANH, RB, CB, KW, FS_OUT_PACKED, NP, AF>(a, ep, s);
+        return launch_fs<LX_EPI_NONE, RB, CB, KW, FS_OUT_PACKED, NP, AF>(a, ep, s);
+      }
+    if (ep.kind == LX_EPI_NONE)
+      return launch_fs<LX_EPI_NONE, RB, CB, KW, FS_OUT_F32, NP, AF>(a, ep, s);
+    if (ep.kind == LX_EPI_GELU_TANH)
+      return launch_fs<LX_EPI_GELU_TANH, RB, CB, KW, FS_OUT_F32, NP, AF>(a, ep, s);
   }
   switch (ep.kind) {
     case LX_EPI_ROPE_PARTIAL:
@@ -264,7 +288,45 @@ bool pick_fs(const FsArgs& a, int out, const EpiArgs& ep, hipStream_t s, int* rc
   return true;
 }
 
+// fp32 or packed rows: one 32 x 32 tile per CU at most, else 32 x 64 (six products, whose
+// loads have twice the MFMAs to hide behind, half a tile more).  N = K = 1024: 148 rows
+// 14.3 -> 8.0 us, 512 rows 14.7 -> 12.3; N = 3072: 148 rows 19.4 -> 14.3, 200 rows (336
+// tiles) 19.3 -> 20.6 and left alone; six products N = 1024, K = 2048, 148 rows 35 -> 16 us.
+template <int NP, int AF>
+bool pick_fs_rows(const FsArgs& a, int out, const EpiArgs& ep, hipStream_t s, int* rc) {
+  const long nrb = (a.M + 31) / 32;
+  if (nrb * (a.N / 32) <= 256)
+    *rc = dispatch_fs<1, 1, 4, NP, AF>(a, out, ep, s);
+  else if (nrb * (a.N / 64) <= (NP == 3 ? 256 : 384))
+    *rc = dispatch_fs<1, 2, 4, NP, AF>(a, out, ep, s);
+  else
+    return false;
+  return true;
+}
+
 }  // namespace
+
+bool linear_fs_rows(const lx_linear_bx& g, const EpiArgs& ep, hipStream_t stream, int* rc) {
+  const size_t ab = ((size_t)(g.M - 1) * g.lda + g.K) * 4, wb = (size_t)g.N * g.K * 6;
+  if (ep.kind == LX_EPI_SWIGLU_PAIRED || ab >= (1ull << 31) || wb >= (1ull << 31)) return false;
+  FsArgs a{};
+  a.A = g.A;
+  a.lda = g.lda;
+  a.a_bytes = (unsigned)ab;
+  a.Wf = g.Wf;
+  a.w_bytes = (unsigned)wb;
+  a.bias = g.bias;
+  a.Y = g.Y;
+  a.ldy = g.ldy;
+  a.M = g.M;
+  a.N = g.N;
+  a.K = g.K;
+  a.slices = 1;
+  const int out = g.out == LX_BX_OUT_PACKED ? FS_OUT_PACKED : FS_OUT_F32;
+  if (g.a_packed) return pick_fs_rows<3, kAPacked>(a, out, ep, stream, rc);
+  return g.products == 3 ? pick_fs_rows<3, kARows>(a, out, ep, stream, rc)
+                         : pick_fs_rows<6, kARows>(a, out, ep, stream, rc);
+}
 
 int linear_fs(const FsLinear& g, hipStream_t stream) {
   const int npl = g.products == 6 ? 3 : 2;

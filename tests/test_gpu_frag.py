@@ -71,3 +71,33 @@ def test_prefill_projection_tiles_vs_oracle(gpu, qwen2, L, products):
         assert orc.rel_err(k[:L].cpu().numpy(), o.k_cache[layer, :L]) < tol, layer
         assert orc.rel_err(v[:L].cpu().numpy(), o.v_cache[layer, :L]) < tol, layer
     assert orc.rel_err(logits.cpu().numpy(), rl) < tol
+
+
+@pytest.mark.parametrize("M,N,K,products,lda", [
+    (1, 1024, 1024, 3, 0), (33, 1024, 2048, 6, 0), (85, 3072, 1024, 3, 0), (86, 3072, 1024, 3, 12),
+    (256, 1024, 1024, 3, 0), (257, 1024, 1024, 6, 4), (512, 1024, 64, 3, 0), (31, 128, 64, 6, 0),
+    (256, 3072, 128, 6, 0),
+])
+def test_linear_bx_few_rows(gpu, M, N, K, products, lda):
+    """lx_linear_bx on fp32 rows at the row counts of the few-row kernel (row strides past K
+    among them), against float64: each operand is its two or three bf16 parts (2^-17 or 2^-25
+    of it at most, signs at random), the rest fp32 sums."""
+    from larynx_amd import ops
+    announce(f"linear_bx few rows M={M} N={N} K={K} products={products}")
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K + lda, generator=g)[:, :K]
+    W, b = torch.randn(N, K, generator=g) / K ** 0.5, torch.randn(N, generator=g)
+    h = torch.randn(M, N, generator=g)
+    xd = torch.zeros(M, K + lda, device=gpu)
+    xd[:, :K] = x.to(gpu)
+    wf = ops.wfrag_pack(W.to(gpu))
+    y0 = x.double() @ W.double().t() + b.double()
+    tol = 1e-5 if products == 3 else 1e-6
+    cases = ((None, y0, None), (ops.LX_EPI_RESID, h.double() + y0, h),
+             (ops.LX_EPI_GELU_TANH, torch.nn.functional.gelu(y0, approximate="tanh"), None))
+    for kind, ref, init in cases:
+        ep = ops.Epilogue(kind=kind) if kind is not None else None
+        out = init.to(gpu) if init is not None else None
+        y = ops.linear_bx(xd[:, :K], wf, N, b.to(gpu), ep, out=out, bm=64, products=products)
+        err = ((y.cpu().double() - ref).norm() / ref.norm()).item()
+        assert err < tol, (kind, err)
