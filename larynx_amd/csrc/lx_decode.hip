@@ -12,7 +12,8 @@
 //     cache append (src/llm/llm.cpp:200-204) happen in the QKV epilogue;
 //   - silu(gate) * up (src/llm/llm.cpp:284-288) in the gate/up epilogue;
 //   - the residual adds (src/llm/llm.cpp:281, 289) in the o / down epilogues.
-// Attention over the cache is split-key GQA: one workgroup per (64-key split,
+// Attention over the cache is split-key GQA past 64 keys (a shorter cache is attended
+// inside the o_proj launch): one workgroup per (64-key split,
 // kv head) scores all query heads of its group; while the whole cache fits one
 // split that pass writes the output, past it every workgroup of the o_proj
 // launch merges the partial softmax states itself before its rows (five
@@ -415,6 +416,102 @@ __global__ __launch_bounds__(64 * kMergeWaves) void dec_merge_o_kernel(DecAttnAr
   if (row < o.N && lane == 0) o.y[row] = res + v;
 }
 
+// Attention of a short cache fused into o_proj + residual: while the keys fit one
+// 64-key tile, every workgroup of the o_proj launch forms the whole attention row
+// itself from the tiles of the two kv heads (64 KB, read from L2 by 112 workgroups at
+// hidden 896), which takes less than a launch of its own (cache 30: 598 -> 578 us per token).  Wave w takes
+// query heads 2 (w % 4) and 2 (w % 4) + 1 of kv head w / 4, so a K or V row read from LDS
+// serves two heads (one head per wave read twice as much and gained half): lane = key
+// for the scores, lane = (key group, channel quad) for P V, the groups added by the
+// half-wave swaps.  It owns o_proj row 8 * blockIdx.x + w, whose weights are requested
+// before the first wait.
+constexpr int kFuseWaves = 8;
+
+template <int NL>
+__global__ __launch_bounds__(64 * kFuseWaves) void dec_attn_o_kernel(DecAttnArgs at,
+                                                                     DecGemvArgs o) {
+  constexpr int IT = 2 * kKeys * (kHD / 4) / (64 * kFuseWaves);  // tile float4 per thread
+  __shared__ __attribute__((aligned(16))) float ks[2 * kKeys][kHD + 4];
+  __shared__ __attribute__((aligned(16))) float vs[2 * kKeys][kHD];
+  __shared__ float4 qs[2 * kMaxRep * kHD / 4], xs[2 * kMaxRep * kHD / 4];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int NH = at.n_heads;
+  float4 kt[IT], vt[IT];
+#pragma unroll
+  for (int i = 0; i < IT; ++i) {
+    const int idx = tid + 64 * kFuseWaves * i, row = idx >> 4, c4 = idx & 15;
+    const long off = (long)min(row % kKeys, at.max_rows - 1) * at.ld + row / kKeys * kHD + c4 * 4;
+    kt[i] = *reinterpret_cast<const float4*>(at.k_cache + off);
+    vt[i] = *reinterpret_cast<const float4*>(at.v_cache + off);
+  }
+  float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (tid < NH * (kHD / 4)) q = reinterpret_cast<const float4*>(at.q)[tid];
+  const int Tk = *at.pos + 1;
+  const long row = (long)blockIdx.x * kFuseWaves + wave;
+  const long rc = min(row, o.N - 1);
+  const int K4 = o.K >> 2;
+  const float4* W4 = reinterpret_cast<const float4*>(o.W) + rc * K4;
+  float4 w[NL];
+#pragma unroll
+  for (int j = 0; j < NL; ++j) w[j] = ld_nt(W4 + min(lane + j * 64, K4 - 1));
+  const float res = o.y[rc];
+#pragma unroll
+  for (int i = 0; i < IT; ++i) {
+    const int idx = tid + 64 * kFuseWaves * i, kr = idx >> 4, c4 = idx & 15;
+    *reinterpret_cast<float4*>(&ks[kr][c4 * 4]) = kt[i];
+    // rows past the keys may hold anything; their weight is zero
+    *reinterpret_cast<float4*>(&vs[kr][c4 * 4]) =
+        kr % kKeys < Tk ? vt[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  if (tid < NH * (kHD / 4))
+    qs[tid] = make_float4(q.x * at.scale, q.y * at.scale, q.z * at.scale, q.w * at.scale);
+  __syncthreads();
+  const int g = wave >> 2, hr = 2 * (wave & 3);
+  if (hr < at.rep) {
+    // the second head repeats the first where the group has an odd one (not stored)
+    const int h0 = g * at.rep + hr, h1 = g * at.rep + min(hr + 1, at.rep - 1);
+    float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kHD / 4; ++j) {
+      const float4 k4 = *reinterpret_cast<const float4*>(&ks[g * kKeys + lane][4 * j]);
+      s0 += dot4(k4, qs[h0 * (kHD / 4) + j]);
+      s1 += dot4(k4, qs[h1 * (kHD / 4) + j]);
+    }
+    const bool live = lane < Tk;
+    const float m0 = wave_max(live ? s0 : -INFINITY), m1 = wave_max(live ? s1 : -INFINITY);
+    const float p0 = live ? expf(s0 - m0) : 0.0f, p1 = live ? expf(s1 - m1) : 0.0f;
+    const float l0 = wave_sum(p0), l1 = wave_sum(p1);
+    const int kg = lane >> 4, c4 = lane & 15;
+    float4 a0 = make_float4(0.f, 0.f, 0.f, 0.f), a1 = a0;
+    const int nj = min(16, (Tk + 3) >> 2);  // quads of keys
+    for (int j = 0; j < nj; ++j) {
+      const int key = kg + 4 * j;
+      const float w0 = __shfl(p0, key, 64), w1 = __shfl(p1, key, 64);
+      const float4 v = *reinterpret_cast<const float4*>(&vs[g * kKeys + key][4 * c4]);
+      a0 = make_float4(a0.x + w0 * v.x, a0.y + w0 * v.y, a0.z + w0 * v.z, a0.w + w0 * v.w);
+      a1 = make_float4(a1.x + w1 * v.x, a1.y + w1 * v.y, a1.z + w1 * v.z, a1.w + w1 * v.w);
+    }
+    auto groups = [](float x) {
+      x += lane_xor16(x);
+      return x + lane_xor32(x);
+    };
+    a0 = make_float4(groups(a0.x), groups(a0.y), groups(a0.z), groups(a0.w));
+    a1 = make_float4(groups(a1.x), groups(a1.y), groups(a1.z), groups(a1.w));
+    if (kg == 0) xs[h0 * (kHD / 4) + c4] = make_float4(a0.x / l0, a0.y / l0, a0.z / l0, a0.w / l0);
+    if (kg == 1 && h1 != h0)
+      xs[h1 * (kHD / 4) + c4] = make_float4(a1.x / l1, a1.y / l1, a1.z / l1, a1.w / l1);
+  }
+  __syncthreads();
+  float acc = 0.0f;
+#pragma unroll
+  for (int j = 0; j < NL; ++j) {
+    const int k4 = lane + j * 64;
+    if (k4 < K4) acc += dot4(w[j], xs[k4]);
+  }
+  const float v = wave_sum(acc);
+  if (row < o.N && lane == 0) o.y[row] = res + v;
+}
+
 // Writes the position and the token's embedding row (bit-exact copy).
 __global__ __launch_bounds__(256) void dec_begin_kernel(const float* __restrict__ table, long row,
                                                         int D4, float* __restrict__ x, int* d_pos,
@@ -494,6 +591,22 @@ int dec_attention(const DecAttnArgs& a, int n_kv_heads, hipStream_t s) {
   // workgroups write the normalised output
   hipLaunchKernelGGL(dec_attn_partial_kernel, dim3(1, n_kv_heads), dim3(256), 0, s, a);
   return check_launch("dec_attn_partial_kernel");
+}
+
+bool dec_attention_fused(int n_kv_heads, int n_heads) {
+  return n_kv_heads == 2 && n_heads <= 2 * kMaxRep;
+}
+
+int dec_attention_short(const DecAttnArgs& a, int n_kv_heads, const DecGemvArgs& o,
+                        hipStream_t s) {
+  LX_REQUIRE(dec_attention_fused(n_kv_heads, a.n_heads) && a.n_heads == n_kv_heads * a.rep &&
+                 a.ld % 4 == 0 && a.max_rows >= 1 && o.W && o.y && o.N > 0 &&
+                 o.K == a.n_heads * kHD,
+             "dec_attention_short: bad args");
+  static_assert(2 * kMaxRep * kHD <= 1024, "four float4 of an o_proj row per lane");
+  hipLaunchKernelGGL(dec_attn_o_kernel<4>, dim3((unsigned)((o.N + kFuseWaves - 1) / kFuseWaves)),
+                     dim3(64 * kFuseWaves), 0, s, a, o);
+  return check_launch("dec_attn_o_kernel");
 }
 
 template <int SPL, int NL>

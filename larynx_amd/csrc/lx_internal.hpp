@@ -242,6 +242,11 @@ struct DecAttnArgs {
 // Position + 1 <= dec_attention_split_keys(): one launch over the single
 // split, writing the normalised output.
 int dec_attention(const DecAttnArgs& a, int n_kv_heads, hipStream_t stream);
+// The same with the attention formed inside the o_proj + residual launch (o: DEC_RESID
+// arguments, x unused), where dec_attention_fused.
+bool dec_attention_fused(int n_kv_heads, int n_heads);
+int dec_attention_short(const DecAttnArgs& a, int n_kv_heads, const DecGemvArgs& o,
+                        hipStream_t s);
 // Longer caches: the split partial pass, then the merge fused into o_proj +
 // residual (o: DEC_RESID arguments, x unused).  Split class `cls` covers up to
 // the cls-th split count; dec_attention_class(n_split) picks it (-1: past

@@ -313,11 +313,11 @@ int prefill_layer(lx_qwen2* m, Layer& L, int rows, const float* next_norm, hipSt
 
 // One decode layer (src/llm/llm.cpp:254-289): RMSNorm + QKV + rotary + cache
 // append; attention; o_proj + residual; RMSNorm + gate/up + SwiGLU;
-// down_proj + residual.  While the cache fits one split (cls 0) the attention
-// is one launch writing its output and o_proj a launch of its own; past it
-// (cls = 1 + split class) the split partials are merged inside the o_proj
-// launch: five launches per layer either way.  The position is read from
-// m->d_pos.
+// down_proj + residual.  While the cache fits one split (cls 0) the attention is
+// formed inside the o_proj launch (four launches per layer; geometries that kernel
+// does not cover take a launch each); past it (cls = 1 + split class) the split
+// partials are a launch of their own and merged inside o_proj's.  The position is
+// read from m->d_pos.
 int decode_layer(lx_qwen2* m, Layer& L, int cls, hipStream_t s) {
   const int H = m->H, KV = m->KV;
   DecGemvArgs q;
@@ -356,7 +356,9 @@ int decode_layer(lx_qwen2* m, Layer& L, int cls, hipStream_t s) {
   o.y = m->x;
   o.N = H;
   o.K = H;
-  if (cls == 0) {
+  if (cls == 0 && dec_attention_fused(m->NKV, m->NH)) {
+    LX_TRY(dec_attention_short(at, m->NKV, o, s));
+  } else if (cls == 0) {
     LX_TRY(dec_attention(at, m->NKV, s));
     LX_TRY(dec_gemv(DEC_RESID, o, s));
   } else {
@@ -389,7 +391,9 @@ int decode_stack(lx_qwen2* m, int cls, hipStream_t s) {
 // fit one attention split, else 1 + the split class of their split count.
 int decode_class(int pos) {
   const int n_split = (pos + 1 + dec_attention_split_keys() - 1) / dec_attention_split_keys();
-  return n_split == 1 ? 0 : 1 + dec_attention_class(n_split);
+  if (n_split == 1) return 0;
+  const int c = dec_attention_class(n_split);
+  return c < 0 ? -1 : 1 + c;
 }
 
 // Captures the decode layer stack into a HIP graph on the library's own
