@@ -180,6 +180,52 @@ int prefill_partials(lx_qwen2* m, const float* x, int ldx, const void* wf, const
   return gemm_splitk_partials(x, ldx, w, K, m->ws, rows, N, K, *splits, ks, s);
 }
 
+// Gate/up with SwiGLU, down_proj as K-slice partials, residual + next_norm (in
+// out_form) on fp32 activations; hn_form: m->hn as fp32 or two-part packed rows.
+int prefill_mlp(lx_qwen2* m, Layer& L, int rows, const float* next_norm, hipStream_t s,
+                int hn_form, int out_form) {
+  const int H = m->H;
+  lx_epilogue swiglu{};
+  swiglu.kind = LX_EPI_SWIGLU_PAIRED;
+  if (m->frag) {
+    // gate/up + SwiGLU: 64-row tiles with the split tail where it applies (L =
+    // 256: 304 tiles, 256 whole and 48 in five k ranges; 24.3 vs 25.3 us on
+    // 128-row tiles with cold weights), else 128-row tiles while they fit one
+    // round over the CUs, else 64-row tiles (L = 1024: 95 vs 116 us)
+    const bool split = bx_split_parts(rows, 2 * m->I, H, 64) > 0;
+    lx_linear_bx g{};
+    if (split) {
+      g.split_tail = 1;
+      g.ws = m->ws;
+      g.ws_floats = m->ws_floats;
+      g.counters = m->arrivals;
+      g.n_counters = m->n_arrivals;
+    }
+    g.A = m->hn;
+    g.a_packed = hn_form == LX_ACT_PACKED ? 1 : 0;
+    g.lda = H;
+    g.Wf = L.gu_wf;
+    g.epi = &swiglu;
+    g.out = LX_BX_OUT_F32;
+    g.Y = m->act;
+    g.ldy = m->I;
+    g.M = rows;
+    g.N = 2 * m->I;
+    g.K = H;
+    g.bm = split ? 64 : (long)((rows + 127) / 128) * (2 * m->I / 128) <= 256 ? 128 : 64;
+    g.slices = 1;
+    g.products = m->products;
+    LX_TRY(linear_bx(g, s));
+  } else {
+    LX_TRY(linear_split_tail(m->hn, H, L.gu_w, nullptr, m->act, m->I, rows, 2 * m->I, H,
+                             &swiglu, m->ws, m->ws_floats, m->arrivals, m->n_arrivals, s));
+  }
+  int sp = 0;
+  LX_TRY(prefill_partials(m, m->act, m->I, L.down_wf, L.down_w, rows, H, m->I, &sp, s));
+  return splitk_resid_rmsnorm(m->ws, sp, rows, H, nullptr, m->x, next_norm, m->eps, m->hn, s,
+                              out_form);
+}
+
 // Prefill layer (src/llm/llm.cpp:141-173) over L rows at positions m->pos[0..L).
 // On entry m->hn holds input_layernorm(x); on exit x is the layer output and
 // m->hn holds next_norm(x) (the next layer's input_layernorm or the final norm).
@@ -191,6 +237,9 @@ int prefill_partials(lx_qwen2* m, const float* x, int ldx, const void* wf, const
 //   down_proj: K-slice partials, then residual + next_norm in one pass.
 // Every GEMM input (the RMSNorms' and attention's output, SwiGLU's) is written in
 // fragment order by its producer; the last norm is fp32 (the logits GEMM reads it).
+// Where 128-row tiles pad the rows by a tenth or more past one round of the CUs (L =
+// 400: 304 gate/up tiles, a quarter of their rows padding, 42.6 us against 36.9), the
+// MLP runs on the 64-row tiles of the split-operand GEMM instead.
 int prefill_layer_frag(lx_qwen2* m, Layer& L, int rows, const float* next_norm, hipStream_t s,
                        bool last) {
   const int H = m->H, KV = m->KV, QKV = m->QKV;
@@ -228,6 +277,13 @@ int prefill_layer_frag(lx_qwen2* m, Layer& L, int rows, const float* next_norm, 
   o.N = H;
   o.K = H;
   LX_TRY(linear_fs(o, s));
+  const long wide = (rows + 127) / 128;
+  if (m->products == 3 && wide * (2 * m->I / 128) > 256 && rows <= 1024 &&
+      wide * 128 * 10 > (long)rows * 11) {
+    LX_TRY(splitk_resid_rmsnorm(nullptr, 0, rows, H, nullptr, m->x, L.post_norm, m->eps, m->hn, s,
+                                LX_ACT_PACKED));
+    return prefill_mlp(m, L, rows, next_norm, s, LX_ACT_PACKED, last ? LX_ACT_F32 : form);
+  }
   LX_TRY(splitk_resid_rmsnorm(nullptr, 0, rows, H, nullptr, m->x, L.post_norm, m->eps, m->hn, s,
                               form));
   lx_epilogue swiglu{};
@@ -273,42 +329,7 @@ int prefill_layer(lx_qwen2* m, Layer& L, int rows, const float* next_norm, hipSt
                    LX_ACT_F32, s));
   LX_TRY(prefill_partials(m, m->att, H, L.o_wf, L.o_w, rows, H, H, &sp, s));
   LX_TRY(splitk_resid_rmsnorm(m->ws, sp, rows, H, nullptr, m->x, L.post_norm, m->eps, m->hn, s));
-  lx_epilogue swiglu{};
-  swiglu.kind = LX_EPI_SWIGLU_PAIRED;
-  if (m->frag) {
-    // gate/up + SwiGLU: 64-row tiles with the split tail where it applies (L =
-    // 256: 304 tiles, 256 whole and 48 in five k ranges; 24.3 vs 25.3 us on
-    // 128-row tiles with cold weights), else 128-row tiles while they fit one
-    // round over the CUs, else 64-row tiles (L = 1024: 95 vs 116 us)
-    const bool split = bx_split_parts(rows, 2 * m->I, H, 64) > 0;
-    lx_linear_bx g{};
-    if (split) {
-      g.split_tail = 1;
-      g.ws = m->ws;
-      g.ws_floats = m->ws_floats;
-      g.counters = m->arrivals;
-      g.n_counters = m->n_arrivals;
-    }
-    g.A = m->hn;
-    g.lda = H;
-    g.Wf = L.gu_wf;
-    g.epi = &swiglu;
-    g.out = LX_BX_OUT_F32;
-    g.Y = m->act;
-    g.ldy = m->I;
-    g.M = rows;
-    g.N = 2 * m->I;
-    g.K = H;
-    g.bm = split ? 64 : (long)((rows + 127) / 128) * (2 * m->I / 128) <= 256 ? 128 : 64;
-    g.slices = 1;
-    g.products = m->products;
-    LX_TRY(linear_bx(g, s));
-  } else {
-    LX_TRY(linear_split_tail(m->hn, H, L.gu_w, nullptr, m->act, m->I, rows, 2 * m->I, H,
-                             &swiglu, m->ws, m->ws_floats, m->arrivals, m->n_arrivals, s));
-  }
-  LX_TRY(prefill_partials(m, m->act, m->I, L.down_wf, L.down_w, rows, H, m->I, &sp, s));
-  return splitk_resid_rmsnorm(m->ws, sp, rows, H, nullptr, m->x, next_norm, m->eps, m->hn, s);
+  return prefill_mlp(m, L, rows, next_norm, s, LX_ACT_F32, LX_ACT_F32);
 }
 
 // One decode layer (src/llm/llm.cpp:254-289): RMSNorm + QKV + rotary + cache

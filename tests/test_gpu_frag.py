@@ -51,7 +51,8 @@ def qwen2(gpu):
 
 
 @pytest.mark.parametrize("L,products", [
-    (1, 6), (31, 3), (32, 3), (33, 6), (65, 3), (129, 3), (129, 6), (545, 3), (1089, 3),
+    (1, 6), (31, 3), (32, 3), (33, 6), (65, 3), (129, 3), (129, 6), (385, 3), (545, 3), (640, 3),
+    (1089, 3),
 ])
 def test_prefill_projection_tiles_vs_oracle(gpu, qwen2, L, products):
     """q|k|v with the rotary and cache append in its epilogue, o_proj's residual epilogue,
