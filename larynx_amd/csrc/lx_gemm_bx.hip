@@ -590,8 +590,10 @@ int launch_bx(const BxArgs& a, const EpiArgs& ep, hipStream_t stream) {
 // BX_OUT_PACKED on 64-row tiles; the host checks this).
 template <int BMB, int NP, int AP = 0>
 int dispatch_bx(const BxArgs& a, int out, const EpiArgs& ep, hipStream_t s) {
-  if (out == BX_OUT_PARTIAL) return launch_bx<LX_EPI_NONE, BMB, BX_OUT_PARTIAL, NP, AP>(a, ep, s);
-  if constexpr (BMB == 2 && NP == 3) {
+  if constexpr (BMB != 3)
+    if (out == BX_OUT_PARTIAL)
+      return launch_bx<LX_EPI_NONE, BMB, BX_OUT_PARTIAL, NP, AP>(a, ep, s);
+  if constexpr (BMB != 4 && NP == 3) {
     if (out == BX_OUT_PACKED) {
       if (ep.kind == LX_EPI_GELU_TANH)
         return launch_bx<LX_EPI_GELU_TANH, BMB, BX_OUT_PACKED, NP, AP>(a, ep, s);
@@ -754,6 +756,19 @@ int linear_bx(const lx_linear_bx& g, hipStream_t stream) {
       a.ws_bytes = (int)(need * 4);
       a.counters = g.counters;
     }
+  }
+  // More rows than one 64-row tile per CU holds leave some CUs with two tiles, which take
+  // half as long again: 96-row tiles end sooner while one per CU holds them (M = 1040, N =
+  // 2048 26.1 -> 22.5 us, six products 40.3 -> 34.7; M = 768, N = 3072 29.0 -> 27.7 / 43.7 ->
+  // 38.4; M = 666, N = 3072, whose 264 tiles hold less than 256 tiles' rows, 26.2 / 27.1
+  // and kept).  Each element's sums keep their order.
+  const long t96 = (long)((g.M + 95) / 96) * a.tiles_n;
+  if (!a.streamk && slices == 1 && g.out != BX_OUT_PARTIAL && g.bm == 64 &&
+      (long)g.M * a.tiles_n > 64L * device_cus() && t96 <= device_cus()) {
+    a.tiles_m = (g.M + 95) / 96;
+    if (g.a_packed) return dispatch_bx<3, 3, 1>(a, g.out, ep, stream);
+    return g.products == 3 ? dispatch_bx<3, 3>(a, g.out, ep, stream)
+                           : dispatch_bx<3, 6>(a, g.out, ep, stream);
   }
   if (g.a_packed)
     return g.bm == 128 ? dispatch_bx<4, 3, 1>(a, g.out, ep, stream)
