@@ -40,10 +40,10 @@ constexpr int kSolveChunk = 16;    // solve steps whose modulations one GEMV com
 // 64-row tiles number 128, half the CUs.
 constexpr int kPartialRows = 1024;
 // Up to this many rows the block runs on the fragment-operand GEMMs (linear_fs)
-// with three and with six products.  One evaluation at B = 2: T = 24 2014 -> 1317
-// us, T = 74 1985 -> 1489, T = 160 2188 -> 1845, T = 256 2207 -> 2066 (T = 300 2368 /
+// with three and with six products.  One evaluation at B = 2: T = 24 2014 -> 1296
+// us, T = 74 1985 -> 1303, T = 160 2168 -> 1816, T = 256 2195 -> 2033 (T = 300 2368 /
 // 2389: even, and the larger launches keep the split tail); six products T = 24
-// 2413 -> 1622, T = 160 2573 -> 2445, T = 211 (422 rows) slower.
+// 2413 -> 1602, T = 160 2573 -> 2422, T = 211 (422 rows) slower.
 constexpr int kFragRows3 = 512;
 constexpr int kFragRows6 = 320;
 
@@ -204,7 +204,7 @@ int forward_core(lx_dit* m, const float* x, long x_bstride, const float* mu, con
   // the QKV projection's 384 tiles run 256 whole and 128 in two k ranges).
   auto proj = [&](const float* x, int ldx, const void* Wf, const float* W, const float* bias,
                   float* y, int ldy, int N, int K, const lx_epilogue* epi,
-                  bool pack_out = false, int pack_from = 0) -> int {
+                  bool pack_out = false, int pack_from = 0, const FsLn* ln = nullptr) -> int {
     if (!m->frag) return lx_linear_f32(x, ldx, W, bias, y, ldy, rows, N, K, epi, s);
     if (fs) {
       FsLinear f;
@@ -220,7 +220,7 @@ int forward_core(lx_dit* m, const float* x, long x_bstride, const float* mu, con
       f.K = K;
       f.products = m->products;
       f.pack_from = pack_from;
-      return linear_fs(f, s);
+      return ln ? linear_fs_ln(f, *ln, s) : linear_fs(f, s);
     }
     lx_linear_bx g{};
     if (m->qkv_ws) {
@@ -297,7 +297,12 @@ int forward_core(lx_dit* m, const float* x, long x_bstride, const float* mu, con
     const float* w2 = m->frag ? nullptr : m->ff0_w[i];
     const float* w3 = m->frag ? nullptr : m->ff2_w[i];
 
-    LX_TRY(adaln(shift_msa, scale_msa, m->xn, form));
+    // the LayerNorm inside the projection's launch where that takes it
+    const FsLn ln1{m->h, shift_msa, scale_msa, NA, T, kLnEps};
+    const FsLn ln2{m->h, shift_mlp, scale_mlp, NA, T, kLnEps};
+    const bool in1 = fs && !pk_kv && fs_takes_ln(rows, 3 * D, D, m->products);
+    const bool in2 = fs && fs_takes_ln(rows, m->F, D, m->products);
+    if (!in1) LX_TRY(adaln(shift_msa, scale_msa, m->xn, form));
     lx_epilogue rope{};
     rope.kind = LX_EPI_ROPE_PARTIAL;
     rope.rows_per_batch = T;
@@ -307,16 +312,17 @@ int forward_core(lx_dit* m, const float* x, long x_bstride, const float* mu, con
     rope.rope_sections = 2;
     rope.rope_base = kRopeBase;
     LX_TRY(proj(m->xn, D, wf0, w0, m->qkv_b[i], m->qkv, 3 * D, 3 * D, D, &rope, pk_kv,
-                /*pack_from*/ D));
+                /*pack_from*/ D, in1 ? &ln1 : nullptr));
     LX_TRY(attention(m->qkv, 3 * D, m->qkv + D, 3 * D, m->qkv + 2 * D, 3 * D, m->att, D, B, T,
                      T, m->heads, m->heads, m->hd, 1.0f / std::sqrt((float)m->hd), 0, 0,
                      m->products, form, s, pk_kv ? 1 : 0));
     LX_TRY(proj_gated(m->att, D, wf1, w1, m->out_b[i], gate_msa, D));
 
-    LX_TRY(adaln(shift_mlp, scale_mlp, m->xn, form));
+    if (!in2) LX_TRY(adaln(shift_mlp, scale_mlp, m->xn, form));
     lx_epilogue gelu{};
     gelu.kind = LX_EPI_GELU_TANH;
-    LX_TRY(proj(m->xn, D, wf2, w2, m->ff0_b[i], m->ff, m->F, m->F, D, &gelu, /*pack_out*/ true));
+    LX_TRY(proj(m->xn, D, wf2, w2, m->ff0_b[i], m->ff, m->F, m->F, D, &gelu, /*pack_out*/ true,
+                0, in2 ? &ln2 : nullptr));
     LX_TRY(proj_gated(m->ff, m->F, wf3, w3, m->ff2_b[i], gate_mlp, m->F));
     if (m->cap.blocks) {
       if (pending) {  // the block's output: fold the FF2 slices into h now

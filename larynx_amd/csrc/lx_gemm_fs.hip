@@ -221,6 +221,151 @@ int launch_fs(const FsArgs& a, const EpiArgs& ep, hipStream_t s) {
   return check_launch("gemm_fs_kernel");
 }
 
+// The modulated LayerNorm of the block input inside the projection that reads it, for
+// launches of at most one workgroup per CU (three products, rows of 1024): a launch of
+// its own costs 4.5 us at these sizes, nearly all of it latency.  Eight waves own a
+// 32 x 64 tile, an eighth of K each.  Every workgroup normalises its 32 rows itself
+// (four rows per wave, the arithmetic of adaln_kernel), splits them into fragments in LDS
+// (128 KB; the 16-byte slots of a 32-row fragment are XOR-swizzled by k step and half, so
+// that a row's 8-byte stores fall on all banks) and multiplies from there, while its
+// first W fragments are on their way.  The partial tiles then reuse the LDS.  One
+// evaluation at B = 2, T = 50 1406 -> 1299 us, T = 74 1468 -> 1303, T = 128 1785 -> 1434 (FF0's
+// alone there).
+constexpr int kLnK = 1024;
+
+template <int EPI, int OUT>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+gemm_fs_ln_kernel(FsArgs a, EpiArgs ep, FsLn ln) {
+  constexpr int KW = 8, CB = 2, NPL = 2, D = 4, NKS = kLnK / 16, NW = NKS / KW, NV = kLnK / 256;
+  extern __shared__ __attribute__((aligned(16))) float red[];
+  char* fl = reinterpret_cast<char*>(red);  // [NKS][NPL][64] 16-byte slots
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 31, h = lane >> 5;
+  int w = blockIdx.x;
+  {
+    const int full = gridDim.x / 8 * 8;
+    if (w < full) w = (w % 8) * (full / 8) + w / 8;
+  }
+  const int mt = w % a.tiles_m, nt = w / a.tiles_m;
+  const int m0 = mt * 32, n0 = nt * 64;
+  // rows and the first row's modulation ahead of the weights (loads retire in order)
+  floatx4 x[4][NV];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const floatx4* src = reinterpret_cast<const floatx4*>(
+        ln.x + (long)min(m0 + wave + 8 * i, a.M - 1) * kLnK);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) x[i][j] = src[lane + 64 * j];
+  }
+  int batch = min(m0 + wave, a.M - 1) / ln.T;
+  floatx4 sc[NV], sh[NV];
+  auto mods = [&](int b) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      sc[j] = reinterpret_cast<const floatx4*>(ln.scale + b * ln.mod_stride)[lane + 64 * j];
+      sh[j] = reinterpret_cast<const floatx4*>(ln.shift + b * ln.mod_stride)[lane + 64 * j];
+    }
+  };
+  mods(batch);
+  const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<void*>(a.Wf), (short)0, (int)a.w_bytes, 0x00020000);
+  unsigned ow[CB];
+#pragma unroll
+  for (int c = 0; c < CB; ++c)
+    ow[c] = (unsigned)((n0 / 32 + c) * NKS + wave * NW) * 3072 + lane * 16;
+  uintx4_t fw[D][CB][NPL];
+  auto load = [&](int i, int s) {
+#pragma unroll
+    for (int c = 0; c < CB; ++c)
+#pragma unroll
+      for (int p = 0; p < NPL; ++p)
+        fw[i][c][p] =
+            __builtin_amdgcn_raw_buffer_load_b128(wrs, ow[c] + s * 3072 + p * 1024, 0, 0);
+  };
+#pragma unroll
+  for (int i = 0; i < D; ++i) load(i, i);
+  // one epilogue quad per wave
+  constexpr int SL = CB * 4;
+  static_assert(SL == KW, "one quad per wave");
+  const int em = m0 + r, en = n0 + wave % CB * 32 + (wave / CB & 3) * 8 + h * 4;
+  const FsEpiIn pre = fs_epi_load<EPI, OUT>(a, ep, min(em, a.M - 1), en);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int lr = wave + 8 * i, m = min(m0 + lr, a.M - 1);
+    if (m / ln.T != batch) {  // wave-uniform
+      batch = m / ln.T;
+      mods(batch);
+    }
+    float sm = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) sm += (x[i][j][0] + x[i][j][1]) + (x[i][j][2] + x[i][j][3]);
+    const float mean = wave_sum(sm) / (float)kLnK;
+    float q = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const floatx4 d = x[i][j] - mean;
+      q += (d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3]);
+    }
+    const float rstd = 1.0f / sqrtf(wave_sum(q) / (float)kLnK + ln.eps);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const floatx4 o = ((x[i][j] - mean) * rstd) * (1.0f + sc[j]) + sh[j];
+      const int k4 = lane + 64 * j, ks = k4 >> 2, hh = (k4 >> 1) & 1;
+      char* d = fl + ((ks * NPL) * 64 + hh * 32 + (lr ^ ((2 * ks + hh) & 31))) * 16 + (k4 & 1) * 8;
+      const uintx4_t pk = pack2_bf16(o);
+      *reinterpret_cast<uintx2_t*>(d) = uintx2_t{pk[0], pk[1]};
+      *reinterpret_cast<uintx2_t*>(d + 1024) = uintx2_t{pk[2], pk[3]};
+    }
+  }
+  __syncthreads();
+  floatx16 acc[CB];
+#pragma unroll
+  for (int c = 0; c < CB; ++c)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[c][e] = 0.0f;
+#pragma unroll
+  for (int s = 0; s < NW; ++s) {
+    const int ks = wave * NW + s;
+    const char* src = fl + (ks * NPL * 64 + h * 32 + (r ^ ((2 * ks + h) & 31))) * 16;
+    uintx4_t f[NPL];
+#pragma unroll
+    for (int p = 0; p < NPL; ++p) f[p] = *reinterpret_cast<const uintx4_t*>(src + p * 1024);
+    constexpr int kPa[3] = {1, 0, 0}, kPw[3] = {0, 1, 0};
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+      for (int c = 0; c < CB; ++c)
+        acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag_bf(fw[s % D][c][kPw[q]]),
+                                                         frag_bf(f[kPa[q]]), acc[c], 0, 0, 0);
+    if (s + D < NW) load(s % D, s + D);
+  }
+  __syncthreads();  // every wave is past its fragments
+  floatx4* part4 = reinterpret_cast<floatx4*>(red);
+#pragma unroll
+  for (int c = 0; c < CB; ++c)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      part4[(wave * SL + q * CB + c) * 64 + lane] =
+          floatx4{acc[c][4 * q], acc[c][4 * q + 1], acc[c][4 * q + 2], acc[c][4 * q + 3]};
+  __syncthreads();
+  floatx4 t = part4[wave * 64 + lane];
+#pragma unroll
+  for (int g = 1; g < KW; ++g) t += part4[(g * SL + wave) * 64 + lane];
+  if (em < a.M) fs_epilogue<EPI, OUT, NPL>(a, ep, 0, em, en, h, t, pre);
+}
+
+template <int EPI, int OUT>
+int launch_fs_ln(const FsArgs& a, const EpiArgs& ep, const FsLn& ln, hipStream_t s) {
+  auto kern = gemm_fs_ln_kernel<EPI, OUT>;
+  static LdsLimit once;
+  constexpr size_t lds = (size_t)32 * kLnK * 4;
+  const int rc = raise_lds_limit((const void*)kern, lds, once, "linear_fs_ln");
+  if (rc) return rc;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(512), lds, s, a, ep, ln);
+  return check_launch("gemm_fs_ln_kernel");
+}
+
 template <int RB, int CB, int KW, int NP, int AF>
 int dispatch_fs(FsArgs a, int out, const EpiArgs& ep, hipStream_t s) {
   a.tiles_m = (a.M + 32 * RB - 1) / (32 * RB);
@@ -326,6 +471,42 @@ bool linear_fs_rows(const lx_linear_bx& g, const EpiArgs& ep, hipStream_t stream
   if (g.a_packed) return pick_fs_rows<3, kAPacked>(a, out, ep, stream, rc);
   return g.products == 3 ? pick_fs_rows<3, kARows>(a, out, ep, stream, rc)
                          : pick_fs_rows<6, kARows>(a, out, ep, stream, rc);
+}
+
+// From 65 rows (two row blocks leave the 32 x 64 tiles at 96 workgroups for q|k|v: T =
+// 24 1313 against 1296 us an evaluation) to one workgroup per CU.
+bool fs_takes_ln(int M, int N, int K, int products) {
+  return products == 3 && K == kLnK && N % 64 == 0 && M > 64 &&
+         (long)((M + 31) / 32) * (N / 64) <= 256;
+}
+
+int linear_fs_ln(const FsLinear& g, const FsLn& ln, hipStream_t stream) {
+  const size_t wb = (size_t)g.N * g.K * 6;
+  LX_REQUIRE(ln.x && ln.shift && ln.scale && ln.T > 0 && g.Wf && g.Y && g.M > 0 &&
+                 fs_takes_ln(g.M, g.N, g.K, g.products) && wb < (1ull << 31) && g.epi &&
+                 (g.epi->kind == LX_EPI_ROPE_PARTIAL || g.epi->kind == LX_EPI_GELU_TANH),
+             "linear_fs_ln: bad arguments (M=%d N=%d K=%d)", g.M, g.N, g.K);
+  FsArgs a{};
+  a.Wf = g.Wf;
+  a.w_bytes = (unsigned)wb;
+  a.bias = g.bias;
+  a.Y = g.Y;
+  a.ldy = g.ldy;
+  a.M = g.M;
+  a.N = g.N;
+  a.K = g.K;
+  a.slices = 1;
+  a.tiles_m = (g.M + 31) / 32;
+  a.tiles_n = g.N / 64;
+  EpiArgs ep;
+  LX_TRY(make_epi(g.epi, g.N, &ep));
+  ep.pack_from = g.pack_from;
+  if (g.epi->kind == LX_EPI_GELU_TANH) {
+    LX_REQUIRE(g.out == FS_OUT_FRAG, "linear_fs_ln: GELU is written in fragment order");
+    return launch_fs_ln<LX_EPI_GELU_TANH, FS_OUT_FRAG>(a, ep, ln, stream);
+  }
+  LX_REQUIRE(g.out == FS_OUT_F32, "linear_fs_ln: rotary rows are fp32");
+  return launch_fs_ln<LX_EPI_ROPE_PARTIAL, FS_OUT_F32>(a, ep, ln, stream);
 }
 
 int linear_fs(const FsLinear& g, hipStream_t stream) {

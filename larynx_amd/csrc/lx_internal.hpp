@@ -180,6 +180,17 @@ struct FsLinear {
   float *k_cache = nullptr, *v_cache = nullptr;
 };
 int linear_fs(const FsLinear& g, hipStream_t stream);
+// The same with A = LN(x) * (1 + scale) + shift formed inside the launch (g.A unused;
+// row b * T + t takes modulation row b), where fs_takes_ln: rotary fp32 or GELU
+// fragment-order output.
+struct FsLn {
+  const float *x, *shift, *scale;
+  long mod_stride;
+  int T;
+  float eps;
+};
+bool fs_takes_ln(int M, int N, int K, int products);
+int linear_fs_ln(const FsLinear& g, const FsLn& ln, hipStream_t stream);
 // lx_attention_f32 with the split-operand kernel's product count (3 or 6; the
 // fp32 kernel, which small grids run, ignores it); o in out_form (LX_ACT_*).
 int attention(const float* q, int ldq, const float* k, int ldk, const float* v, int ldv, float* o,

@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("B,T,products", [
-    (1, 5, 3), (2, 16, 3), (2, 17, 6), (2, 80, 3), (2, 83, 6), (1, 161, 3), (2, 160, 6),
+    (1, 5, 3), (2, 16, 3), (2, 17, 6), (2, 32, 3), (2, 33, 3), (1, 65, 3), (2, 80, 3), (3, 41, 3),
+    (2, 128, 3), (2, 83, 6), (1, 161, 3), (2, 160, 6),
     (2, 161, 6), (2, 255, 3), (2, 257, 3),
 ])
 def test_dit_projection_tiles_vs_oracle(gpu, B, T, products):
