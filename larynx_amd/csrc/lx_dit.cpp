@@ -436,10 +436,10 @@ extern "C" int lx_dit_create(const lx_dit_weights* w, int B, int max_T, lx_dit**
   m->h = A(rows * D);
   // (fragment order, up to kFragRows3 rows, takes half as much again)
   const size_t frows = std::min<size_t>(rows, kFragRows3);
-  m->xn = A(std::max(rows * D, act_floats(frows, D)));
+  m->xn = A(std::max(rows * D, act_floats(frows, D, 3)));
   m->qkv = A(rows * 3 * D);
-  m->att = A(std::max(rows * D, act_floats(frows, D)));
-  m->ff = A(std::max(rows * F, act_floats(frows, F)));
+  m->att = A(std::max(rows * D, act_floats(frows, D, 3)));
+  m->ff = A(std::max(rows * F, act_floats(frows, F, 3)));
   m->P = A(rows * mel);
   m->Pws = A(rows * mel * kProjSplitMax);
   m->Rws = m->frag ? A((size_t)2 * std::min<size_t>(rows, kPartialRows) * D) : nullptr;

@@ -11,8 +11,10 @@ namespace lx {
 // Output form of an activation producer: fp32 rows, two-part packed rows
 // (pack2_bf16), or fragment order with two or three bf16 parts (frag_store4).
 enum { LX_ACT_F32 = 0, LX_ACT_PACKED = 1, LX_ACT_FRAG2 = 2, LX_ACT_FRAG3 = 3 };
-// Floats that hold a (rows, K) activation in any form.
-inline size_t act_floats(size_t rows, size_t K) { return (rows + 31) / 32 * 32 * K * 3 / 2; }
+// Floats that hold a (rows, K) activation in every form of at most `parts` bf16 parts.
+inline size_t act_floats(size_t rows, size_t K, int parts) {
+  return (rows + 31) / 32 * 32 * K * parts / 2;
+}
 
 // Device allocations of a composite object (lx_dit, lx_qwen2, lx_flow), made
 // at create time and released together when the object is destroyed.

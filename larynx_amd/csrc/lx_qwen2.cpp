@@ -491,7 +491,7 @@ extern "C" int lx_qwen2_create(const lx_qwen2_weights* w, int max_ctx, lx_qwen2*
   // the fragment-order GEMM needs N multiples of 128 and K of 64 in every
   // prefill projection, and each activation below 2 GiB
   m->frag = QKV % 128 == 0 && H % 128 == 0 && (2 * I) % 128 == 0 && I % 64 == 0 &&
-            act_floats(max_ctx, I) * sizeof(float) < (1ull << 31);
+            act_floats(max_ctx, I, 2) * sizeof(float) < (1ull << 31);
   Arena& a = m->arena;
   bool ok = true;
   auto A = [&](size_t n) {
@@ -522,10 +522,14 @@ extern "C" int lx_qwen2_create(const lx_qwen2_weights* w, int max_ctx, lx_qwen2*
   }
   const size_t rows = max_ctx;
   m->x = A(rows * H);
-  m->hn = A(act_floats(rows, H));
+  // (three-part fragments only up to kFragRows6 rows)
+  auto act = [&](size_t K) {
+    return A(std::max(act_floats(rows, K, 2), act_floats(std::min<size_t>(rows, kFragRows6), K, 3)));
+  };
+  m->hn = act(H);
   m->qkv = A(rows * QKV);
-  m->att = A(act_floats(rows, H));
-  m->act = A(act_floats(rows, I));
+  m->att = act(H);
+  m->act = act(I);
   int tails = 0;
   m->ws_floats = std::max(splitk_ws_floats(max_ctx, H, QKV, I, &tails), bx_split_ws_floats(64));
   m->ws = A(m->ws_floats);
