@@ -139,15 +139,12 @@ def in_step_matrix(records, ops):
     return out
 
 
-def prefill_bx_slices(rows, N, K):
-    """K slices of a Qwen2 prefill projection on the fragment-order GEMM
-    (prefill_bx_slices in larynx_amd/csrc/lx_qwen2.cpp): at most 9 and at most
-    256 / (64-row tiles), then the fewest with the same longest slice."""
-    steps = K // 64
-    tiles = ((rows + 63) // 64) * (N // 128)
-    most = min(9, steps, max(1, 256 // tiles))
-    per = -(-steps // most)
-    return -(-steps // per)
+def prefill_down_slices(rows, N, K):
+    """K slices of the Qwen2 prefill's down_proj (prefill_down_slices in
+    larynx_amd/csrc/lx_qwen2.cpp): about one 32 x 32 tile per CU up to 64 rows, else
+    about one 128 x 128 tile, at most 8 and each at least 512 deep."""
+    tiles = (-(-rows // 32) * (N // 32)) if rows <= 64 else (-(-rows // 128) * (N // 128))
+    return max(1, min(8, K // 512, 256 // tiles))
 
 
 def pack2(torch, x):
@@ -596,21 +593,16 @@ def qwen2_lm(torch, dev, g):
     lm.set_products(3)
     out = {"prefill_L256_ms": round(prefill_ms, 3), "prefill_products": 3,
            "prefill_L256_ms_six_products": round(six_ms, 3), "decode_ms_per_token": {}}
-    L, H, KVW = lm_in.shape[0], cfg.hidden, cfg.n_kv_heads * cfg.head_dim
-    NQKV = H + 2 * KVW
+    L, H = lm_in.shape[0], cfg.hidden
     rec = profiled_kernels(torch, lambda: lm.prefill(lm_in))
-    s_o = prefill_bx_slices(L, H, H)
-    s_d = prefill_bx_slices(L, H, cfg.intermediate)
-    s_q = prefill_bx_slices(L, NQKV, H)
-    # o_proj and down_proj reduce passes alternate within a layer
-    rr = [(s + 3) * L * H * 4 + H * 4 for s in (s_o, s_d)]
+    s_d = prefill_down_slices(L, H, cfg.intermediate)
+    # the first input norm, then per layer the norm after o_proj (its epilogue adds the
+    # residual) and the pass after down_proj
+    norm, down = 2 * L * H * 4 + H * 4, (s_d + 3) * L * H * 4 + H * 4
     out["in_path"] = {
         "resid_rmsnorm_prefill": kernel_gbs(
-            rec, "resid_rmsnorm_kernel", rr,
-            f"L={L}: {s_o} (o_proj) / {s_d} (down_proj) K slices + residual, next RMSNorm"),
-        "qkv_rope_cache_prefill": kernel_gbs(
-            rec, "qkv_rope_cache_kernel", (s_q + 1) * L * NQKV * 4 + NQKV * 4,
-            f"L={L}: {s_q} K slices + bias, NEOX rotary, q out and K/V cache append"),
+            rec, "resid_rmsnorm_kernel", [norm] + [norm, down] * cfg.n_layers,
+            f"L={L}: RMSNorm alone, and {s_d} down_proj K slices + residual + next RMSNorm"),
     }
     weight_bytes = sum(t.numel() for n, t in params.items() if n != "embed_tokens.weight") * 4
     out["decode_stream_gbs"] = {}

@@ -12,12 +12,12 @@
 //     cache append (src/llm/llm.cpp:200-204) happen in the QKV epilogue;
 //   - silu(gate) * up (src/llm/llm.cpp:284-288) in the gate/up epilogue;
 //   - the residual adds (src/llm/llm.cpp:281, 289) in the o / down epilogues.
-// Attention over the cache is split-key GQA past 64 keys (a shorter cache is attended
-// inside the o_proj launch): one workgroup per (64-key split,
-// kv head) scores all query heads of its group; while the whole cache fits one
-// split that pass writes the output, past it every workgroup of the o_proj
-// launch merges the partial softmax states itself before its rows (five
-// launches per layer at every cache length).
+// Attention over a cache of at most 64 keys happens inside the o_proj launch (four
+// launches per layer).  Past that it is split-key GQA: one workgroup per (64-key
+// split, kv head) scores all query heads of its group, and every workgroup of the
+// o_proj launch merges the partial softmax states itself before its rows (five
+// launches per layer).  Geometries the fused launch does not cover run the partial
+// pass on one split too, where it writes the output.
 //
 // The position (= cache length before the token) is read from device memory,
 // so one capture of a layer stack into a HIP graph serves every position.

@@ -2,11 +2,14 @@
 //
 // Host-side counterpart of build_dit / dit_block (src/flow/dit.cpp:34-145) and
 // of the CFM loop of FlowDecoder::infer (src/flow/flow.cpp:202-274).  Instead
-// of a ~8000-node ggml graph the forward is ~10 launches per block:
+// of a ~8000-node ggml graph the forward is seven launches per block:
 //
 //   adaln(x) -> QKV GEMM (+bias, +partial rotary epilogue) -> flash attention
 //   -> out GEMM (+bias, gated-residual epilogue into x) -> adaln(x)
 //   -> FF0 GEMM (+bias, tanh-GELU epilogue) -> FF2 GEMM (+bias, gated residual)
+//
+// or five or six at few rows, where the LayerNorms run inside the GEMMs that read
+// them.
 //
 // and per Euler step the 22 AdaLN modulation linears plus norm_out's are one
 // stacked weight-streaming GEMV (t is shared by both CFG rows and all frames).
@@ -35,8 +38,8 @@ constexpr float kRopeBase = 10000.0f;  // ROPE_FREQ_BASE (src/flow/internal.h:35
 constexpr int kRotDim = 64;        // ROT_DIM (src/flow/internal.h:25)
 constexpr int kProjSplitMax = 9;   // K slices of the proj_out split-K (gemm_splitk_plan's cap)
 constexpr int kSolveChunk = 16;    // solve steps whose modulations one GEMV computes
-// Up to this many rows (B * T) the out and FF2 projections run as two K slices
-// whose sum is folded into the next modulated LayerNorm: at B * T = 1000 their
+// From kFragRows* (below) up to this many rows (B * T) the out and FF2 projections
+// run as two K slices whose sum is folded into the next modulated LayerNorm: at B * T = 1000 their
 // 64-row tiles number 128, half the CUs.
 constexpr int kPartialRows = 1024;
 // Up to this many rows the block runs on the fragment-operand GEMMs (linear_fs)

@@ -52,7 +52,7 @@ def qwen2(gpu):
 
 
 @pytest.mark.parametrize("L,products", [
-    (1, 6), (31, 3), (32, 3), (33, 6), (65, 3), (129, 3), (129, 6), (385, 3), (545, 3), (640, 3),
+    (1, 6), (31, 3), (32, 3), (33, 6), (65, 3), (129, 3), (129, 6), (256, 6), (385, 3), (545, 3), (640, 3),
     (1089, 3),
 ])
 def test_prefill_projection_tiles_vs_oracle(gpu, qwen2, L, products):
