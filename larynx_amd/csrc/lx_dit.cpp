@@ -200,8 +200,7 @@ int forward_core(lx_dit* m, const float* x, long x_bstride, const float* mu, con
   // K and V leave the QKV projection packed too where attention runs on the
   // three-product split kernel (it then stages them without splitting; q
   // stays fp32: attention scales it before its own split).
-  const bool pk_kv =
-      m->frag && m->products == 3 && attention_takes_packed_kv(B, T, m->heads, 3);
+  const bool pk_kv = pk && attention_takes_packed_kv(B, T, m->heads, 3);
   // Every projection on the fragment-order GEMM asks for the split tail: it
   // applies where the launch's tiles number between one and two per CU (T = 500:
   // the QKV projection's 384 tiles run 256 whole and 128 in two k ranges).
@@ -215,14 +214,13 @@ int forward_core(lx_dit* m, const float* x, long x_bstride, const float* mu, con
       f.Wf = Wf;
       f.bias = bias;
       f.epi = epi;
-      f.out = !pack_out ? FS_OUT_F32 : epi->kind == LX_EPI_ROPE_PARTIAL ? FS_OUT_PACKED : FS_OUT_FRAG;
+      f.out = pack_out ? FS_OUT_FRAG : FS_OUT_F32;
       f.Y = y;
       f.ldy = ldy;
       f.M = rows;
       f.N = N;
       f.K = K;
       f.products = m->products;
-      f.pack_from = pack_from;
       return ln ? linear_fs_ln(f, *ln, s) : linear_fs(f, s);
     }
     lx_linear_bx g{};
@@ -303,7 +301,7 @@ int forward_core(lx_dit* m, const float* x, long x_bstride, const float* mu, con
     // the LayerNorm inside the projection's launch where that takes it
     const FsLn ln1{m->h, shift_msa, scale_msa, NA, T, kLnEps};
     const FsLn ln2{m->h, shift_mlp, scale_mlp, NA, T, kLnEps};
-    const bool in1 = fs && !pk_kv && fs_takes_ln(rows, 3 * D, D, m->products);
+    const bool in1 = fs && fs_takes_ln(rows, 3 * D, D, m->products);
     const bool in2 = fs && fs_takes_ln(rows, m->F, D, m->products);
     if (!in1) LX_TRY(adaln(shift_msa, scale_msa, m->xn, form));
     lx_epilogue rope{};

@@ -378,9 +378,6 @@ int dispatch_fs(FsArgs a, int out, const EpiArgs& ep, hipStream_t s) {
         return launch_fs<LX_EPI_GELU_TANH, RB, CB, KW, FS_OUT_FRAG, NP, AF>(a, ep, s);
       return launch_fs<LX_EPI_SWIGLU_PAIRED, RB, CB, KW, FS_OUT_FRAG, NP, AF>(a, ep, s);
     }
-    if constexpr (NP == 3)
-      if (out == FS_OUT_PACKED)
-        return launch_fs<LX_EPI_ROPE_PARTIAL, RB, CB, KW, FS_OUT_PACKED, NP, AF>(a, ep, s);
   }
   if constexpr (AF != kAFrag) {
     if constexpr (NP == 3)
@@ -500,7 +497,6 @@ int linear_fs_ln(const FsLinear& g, const FsLn& ln, hipStream_t stream) {
   a.tiles_n = g.N / 64;
   EpiArgs ep;
   LX_TRY(make_epi(g.epi, g.N, &ep));
-  ep.pack_from = g.pack_from;
   if (g.epi->kind == LX_EPI_GELU_TANH) {
     LX_REQUIRE(g.out == FS_OUT_FRAG, "linear_fs_ln: GELU is written in fragment order");
     return launch_fs_ln<LX_EPI_GELU_TANH, FS_OUT_FRAG>(a, ep, ln, stream);
@@ -520,6 +516,14 @@ int linear_fs(const FsLinear& g, hipStream_t stream) {
   const size_t wb = (size_t)g.N * g.K * 6;
   LX_REQUIRE(ab < (1ull << 31) && wb < (1ull << 31) && (size_t)g.M * g.ldy < (1ull << 40),
              "linear_fs: operands must stay below 2 GiB");
+  const int kind = g.epi ? g.epi->kind : LX_EPI_NONE;
+  LX_REQUIRE(g.neox_pos || g.out == FS_OUT_PARTIAL ||
+                 (g.out == FS_OUT_FRAG
+                      ? kind == LX_EPI_GELU_TANH || kind == LX_EPI_SWIGLU_PAIRED
+                      : g.out == FS_OUT_F32 &&
+                            (kind == LX_EPI_RESID || kind == LX_EPI_GATED_RESID ||
+                             kind == LX_EPI_ROPE_PARTIAL)),
+             "linear_fs: epilogue %d with output %d", kind, g.out);
   FsArgs a{};
   a.A = g.A;
   a.a_bytes = (unsigned)ab;
@@ -535,7 +539,6 @@ int linear_fs(const FsLinear& g, hipStream_t stream) {
   a.slices = g.slices;
   EpiArgs ep;
   LX_TRY(make_epi(g.epi, g.N, &ep));
-  ep.pack_from = g.pack_from;
   if (g.neox_pos) {
     LX_REQUIRE(g.bias && g.rope_cs && g.k_cache && g.v_cache && g.out == FS_OUT_F32 &&
                    g.q_cols % 64 == 0 && g.kv_cols % 64 == 0 && g.q_cols + 2 * g.kv_cols == g.N,

@@ -222,9 +222,6 @@ int dispatch_ft(const FsArgs& a, int out, const EpiArgs& ep, hipStream_t s) {
       return launch_ft<LX_EPI_GELU_TANH, RB, CB, 2, FS_OUT_FRAG, NP>(a, ep, s);
     return launch_ft<LX_EPI_SWIGLU_PAIRED, RB, CB, 2, FS_OUT_FRAG, NP>(a, ep, s);
   }
-  if constexpr (NP == 3)
-    if (out == FS_OUT_PACKED)
-      return launch_ft<LX_EPI_ROPE_PARTIAL, RB, CB, 2, FS_OUT_PACKED, NP>(a, ep, s);
   switch (ep.kind) {
     case LX_EPI_ROPE_PARTIAL:
       return launch_ft<LX_EPI_ROPE_PARTIAL, RB, CB, 2, FS_OUT_F32, NP>(a, ep, s);

@@ -156,24 +156,22 @@ int linear_bx(const lx_linear_bx& g, hipStream_t stream);
 // bm-row tiles (0: the split tail does not apply), and the ws it needs.
 int bx_split_parts(int M, int N, int K, int bm);
 size_t bx_split_ws_floats(int bm);
-// ---- split-operand GEMM for few rows (lx_gemm_fs.hip) ----
-// y = epi(A W^T + bias), A in fragment order (a_frag: LX_ACT_FRAG2 / FRAG3 rows by
-// the product count) or fp32 rows (lda), W = wfrag_pack.  out: FS_OUT_F32 rows,
-// FS_OUT_PACKED two-part packed rows from column pack_from, FS_OUT_FRAG the
-// next projection's fragment-order A (GELU, SWIGLU_PAIRED), FS_OUT_PARTIAL raw
-// products of `slices` K slices.
+// ---- split-operand GEMMs on fragment-order operands (lx_gemm_fs.hip, lx_gemm_ft.hip) ----
+// y = epi(A W^T + bias), A in fragment order (LX_ACT_FRAG2 for three products, FRAG3
+// for six), W = wfrag_pack.  out: FS_OUT_F32 rows (RESID, GATED_RESID, ROPE_PARTIAL),
+// FS_OUT_FRAG the next projection's fragment-order A (GELU_TANH, SWIGLU_PAIRED),
+// FS_OUT_PARTIAL raw products of `slices` K slices.  (FS_OUT_PACKED: lx_linear_bx's
+// packed rows, from fp32 or packed A only.)
 enum { FS_OUT_F32 = 0, FS_OUT_PARTIAL = 1, FS_OUT_PACKED = 2, FS_OUT_FRAG = 3 };
 struct FsLinear {
   const void* A = nullptr;
-  long lda = 0;
-  int a_frag = 1;
   const void* Wf = nullptr;
   const float* bias = nullptr;
   const lx_epilogue* epi = nullptr;
   int out = FS_OUT_F32;
   float* Y = nullptr;
   long ldy = 0, slice_stride = 0;
-  int M = 0, N = 0, K = 0, slices = 1, products = 3, pack_from = 0;
+  int M = 0, N = 0, K = 0, slices = 1, products = 3;
   // q|k|v projection of the LM: bias, NEOX rotary at pos[m] on the first
   // rope_heads heads of 64, q -> Y, k / v -> the caches' row m (kv_cols wide)
   const int* neox_pos = nullptr;
