@@ -576,7 +576,8 @@ __device__ __forceinline__ int vt_pos(int k) {
 // tile t + 2 replaces K of tile t (its scores were formed in iteration t - 1),
 // V of tile t + 1 replaces V of tile t - 1, so one barrier per tile suffices.
 // KVP: K and V arrive as two-part packed rows (their producer split them
-// once; three products), so staging stores the parts without splitting.
+// once; three products), so staging stores the parts without splitting; the output is
+// fp32 or packed rows.
 // OCC = 2: at most 256 registers, so that two 64-query workgroups of three products
 // (72 KB of LDS each) share a CU; the compiler's own choice is above 256, one
 // workgroup per CU, which is a little faster for grids of at most one per CU (T = 500
@@ -980,7 +981,7 @@ __global__ __launch_bounds__(64 * QS * KS) __attribute__((amdgpu_waves_per_eu(OC
           const float mine = keep[i] * a_s, other = part[i * 64 + lane] * a_o;
           w[e] = (ks == 0 ? mine + other : other + mine) * inv;
         }
-        if (opk < LX_ACT_FRAG2)
+        if (KVP || opk < LX_ACT_FRAG2)
           store_o4(o + ((long)b * Tq + qi) * ldo + col + g * 8, w, opk);
         else
           act_store4(o, ldo, b * Tq + qi, col + g * 8, w, opk);
@@ -1043,7 +1044,7 @@ __global__ __launch_bounds__(64 * QS * KS) __attribute__((amdgpu_waves_per_eu(OC
     if (qi < Tq) {
       const float* src = otile + (row >> 5) * (32 * kLD) + (row & 31) * kLD + c;
       const floatx4 w = *reinterpret_cast<const floatx4*>(src);
-      if (opk < LX_ACT_FRAG2)
+      if (KVP || opk < LX_ACT_FRAG2)
         store_o4(o + ((long)b * Tq + qi) * ldo + head * kHD + c, w, opk);
       else
         act_store4(o, ldo, b * Tq + qi, head * kHD + c, w, opk);
@@ -1126,6 +1127,8 @@ int attention(const float* q, int ldq, const float* k, int ldk, const float* v, 
   int np = 0;
   const int layout = attention_layout(B, Tq, n_heads, products, causal, &np);
   // K / V as packed rows: the three-product split kernel only.
+  LX_REQUIRE(!kv_packed || out_form < LX_ACT_FRAG2,
+             "attention: packed K/V write fp32 or packed rows");
   LX_REQUIRE(!kv_packed || np == 3,
              "attention: packed K/V need the three-product split kernel (B=%d Tq=%d)", B, Tq);
   const int qt = layout == 0 ? 32 : layout == 1 ? 64 : 128;
