@@ -659,6 +659,8 @@ int linear_bx(const lx_linear_bx& g, hipStream_t stream) {
              "linear_bx: unknown output %d", g.out);
   LX_REQUIRE(g.a_packed == 0 || g.a_packed == 1, "linear_bx: a_packed=%d must be 0 or 1",
              g.a_packed);
+  LX_REQUIRE(g.split_tail == 0 || g.split_tail == 1, "linear_bx: split_tail=%d must be 0 or 1",
+             g.split_tail);
   LX_REQUIRE((!g.a_packed || g.products == 3) && (g.out != BX_OUT_PACKED ||
                                                    (g.products == 3 && g.bm == 64)),
              "linear_bx: packed operands need three products (the packed output 64-row tiles)");
@@ -720,8 +722,6 @@ int linear_bx(const lx_linear_bx& g, hipStream_t stream) {
   a.counters = nullptr;
   a.split_full = 0;
   a.split_s = 0;
-  LX_REQUIRE(g.split_tail == 0 || g.split_tail == 1, "linear_bx: split_tail=%d must be 0 or 1",
-             g.split_tail);
   if (g.split_tail && g.ws && g.counters && slices == 1 && g.out != BX_OUT_PARTIAL) {
     // whole tiles on the first round of CUs, the rest split along K onto the
     // second, so that no CU holds two whole tiles

@@ -70,7 +70,7 @@ def test_argument_errors_need_no_device():
     # fragment-order GEMM: N not a multiple of 128, an empty last K slice (18
     # steps of 64 as 7 slices of 3), a tile height other than 64 / 128, a
     # product count other than 3 / 6
-    from larynx_amd._lib import LX_BX_OUT_PARTIAL, LinearBx
+    from larynx_amd._lib import LX_BX_OUT_F32, LX_BX_OUT_PARTIAL, LinearBx
     g = LinearBx()
     g.A, g.lda, g.Wf, g.Y, g.ldy, g.M, g.N, g.K, g.bm, g.slices = (16, 1024, 16, 16, 1000,
                                                                    8, 1000, 1024, 64, 1)
@@ -85,6 +85,9 @@ def test_argument_errors_need_no_device():
     assert lib.lx_linear_bx_f32(C.byref(g), None) == LX_ERR_ARG
     assert b"products" in lib.lx_last_error()
     g.products, g.split_tail = 3, 2  # split_tail is a 0 / 1 switch
+    assert lib.lx_linear_bx_f32(C.byref(g), None) == LX_ERR_ARG
+    assert b"split_tail" in lib.lx_last_error()
+    g.out = LX_BX_OUT_F32  # few rows without scratch: a kernel of its own
     assert lib.lx_linear_bx_f32(C.byref(g), None) == LX_ERR_ARG
     assert b"split_tail" in lib.lx_last_error()
     # the folded residual takes at most four partial slices
