@@ -169,3 +169,20 @@ def test_one_hip_runtime_whatever_the_import_order():
                          timeout=300)
     assert out.returncode == 0, out.stderr
     assert out.stdout.strip().splitlines()[-1] == "1"
+
+
+def test_ops_without_the_private_stream_getter():
+    """larynx_amd.ops imports on a torch without the private raw-stream name, and takes the
+    stream from torch's public one."""
+    import subprocess
+    import sys
+    code = ("import types, torch\n"
+            "if hasattr(torch._C, '_cuda_getCurrentRawStream'):\n"
+            "    del torch._C._cuda_getCurrentRawStream\n"
+            "from larynx_amd import ops\n"
+            "torch.cuda.current_stream = lambda: types.SimpleNamespace(cuda_stream=4096)\n"
+            "print(ops.stream().value)\n")
+    out = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True,
+                         timeout=300)
+    assert out.returncode == 0, out.stderr
+    assert out.stdout.strip().splitlines()[-1] == "4096"
