@@ -430,16 +430,18 @@ bool pick_fs(const FsArgs& a, int out, const EpiArgs& ep, hipStream_t s, int* rc
   return true;
 }
 
-// fp32 or packed rows: one 32 x 32 tile per CU at most, else 32 x 64 (six products, whose
-// loads have twice the MFMAs to hide behind, half a tile more).  N = K = 1024: 148 rows
-// 14.3 -> 8.0 us, 512 rows 14.7 -> 12.3; N = 3072: 148 rows 19.4 -> 14.3, 200 rows (336
-// tiles) 19.3 -> 20.6 and left alone; six products N = 1024, K = 2048, 148 rows 35 -> 16 us.
+// fp32 or packed rows: one 32 x 32 tile per CU at most, else one 32 x 64.  N = K = 1024:
+// 148 rows 14.3 -> 8.0 us, 512 rows 14.7 -> 12.3; N = 3072: 148 rows 19.4 -> 14.3, 200 rows
+// (336 tiles) 19.3 -> 20.6 and left alone.  Six products N = 1024, K = 2048: 148 rows 32.1 ->
+// 12.8 us; past one per CU they lose too (N = 896, K = 4864, 768 rows, 336 tiles: 70.1 us on
+// gemm_bx_kernel, 76.9 here; N = 9728, K = 896, 48 rows, 304 tiles: 17.1 / 18.6; N = 3072, K =
+// 1024, 200 rows, 336 tiles: 18.9 / 18.7).
 template <int NP, int AF>
 bool pick_fs_rows(const FsArgs& a, int out, const EpiArgs& ep, hipStream_t s, int* rc) {
   const long nrb = (a.M + 31) / 32;
   if (nrb * (a.N / 32) <= 256)
     *rc = dispatch_fs<1, 1, 4, NP, AF>(a, out, ep, s);
-  else if (nrb * (a.N / 64) <= (NP == 3 ? 256 : 384))
+  else if (nrb * (a.N / 64) <= 256)
     *rc = dispatch_fs<1, 2, 4, NP, AF>(a, out, ep, s);
   else
     return false;

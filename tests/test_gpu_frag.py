@@ -78,7 +78,7 @@ def test_prefill_projection_tiles_vs_oracle(gpu, qwen2, L, products):
 @pytest.mark.parametrize("M,N,K,products,lda", [
     (1, 1024, 1024, 3, 0), (33, 1024, 2048, 6, 0), (85, 3072, 1024, 3, 0), (86, 3072, 1024, 3, 12),
     (256, 1024, 1024, 3, 0), (257, 1024, 1024, 6, 4), (512, 1024, 64, 3, 0), (31, 128, 64, 6, 0),
-    (256, 3072, 128, 6, 0), (700, 3072, 128, 3, 0), (768, 3072, 64, 6, 4), (1040, 2048, 128, 3, 0),
+    (160, 3072, 128, 6, 0), (256, 3072, 128, 6, 0), (700, 3072, 128, 3, 0), (768, 3072, 64, 6, 4), (1040, 2048, 128, 3, 0),
 ])
 def test_linear_bx_few_rows(gpu, M, N, K, products, lda):
     """lx_linear_bx on fp32 rows at the row counts of the few-row kernel (row strides past K
