@@ -12,17 +12,11 @@ from oracle import oracle as orc
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("B,T,products", [
-    (1, 5, 3), (2, 16, 3), (2, 17, 6), (2, 32, 3), (2, 33, 3), (1, 65, 3), (2, 80, 3), (3, 41, 3),
-    (2, 128, 3), (2, 83, 6), (1, 161, 3), (2, 160, 6),
-    (2, 161, 6), (2, 255, 3), (2, 257, 3),
-])
-def test_dit_projection_tiles_vs_oracle(gpu, B, T, products):
-    """Two blocks with O(1) modulation, so that every projection carries weight in the
+def dit_vs_oracle(gpu, cfg, B, T, products):
+    """One evaluation with O(1) modulation, so that every projection carries weight in the
     result.  Tolerance: the two-part operands' 2^-16 per element, some ten roundings deep."""
-    from larynx_amd.flow import DiTConfig, DiTEstimator, dit_param_shapes
-    announce(f"dit B={B} T={T} products={products}")
-    cfg = DiTConfig(depth=2)
+    from larynx_amd.flow import DiTEstimator, dit_param_shapes
+    announce(f"dit F={cfg.ff_inner} B={B} T={T} products={products}")
     params = orc.make_params(dit_param_shapes(cfg), 29)
     dparams = {k: torch.from_numpy(v).to(gpu) for k, v in params.items()}
     est = DiTEstimator(dparams, cfg, B=B, max_T=max(T, 64))
@@ -33,9 +27,31 @@ def test_dit_projection_tiles_vs_oracle(gpu, B, T, products):
     dphi = est.forward(*(torch.from_numpy(a).to(gpu) for a in (x, mu, cond, spks, t)))
     torch.cuda.synchronize()
     est.close()
-    ref = orc.Dit(params, depth=2).forward(x, mu, cond, spks, t)
+    ref = orc.Dit(params, depth=cfg.depth, ff_inner=cfg.ff_inner).forward(x, mu, cond, spks, t)
     err = orc.rel_err(dphi.cpu().numpy(), ref)
     assert err < (1e-4 if products == 3 else 2e-5), err
+
+
+@pytest.mark.parametrize("B,T,products", [
+    (1, 5, 3), (2, 16, 3), (2, 17, 6), (2, 32, 3), (2, 33, 3), (1, 65, 3), (2, 80, 3), (3, 41, 3),
+    (2, 128, 3), (2, 83, 6), (1, 161, 3), (2, 160, 6),
+    (2, 161, 6), (2, 255, 3), (2, 257, 3),
+])
+def test_dit_projection_tiles_vs_oracle(gpu, B, T, products):
+    from larynx_amd.flow import DiTConfig
+    dit_vs_oracle(gpu, DiTConfig(depth=2), B, T, products)
+
+
+@pytest.mark.parametrize("F,B,T,products", [
+    (4096, 2, 37, 6), (4096, 1, 320, 3), (4096, 1, 321, 3), (4096, 2, 128, 6), (4096, 1, 257, 6),
+    (8192, 1, 149, 3), (8192, 1, 289, 3), (8192, 2, 75, 6),
+])
+def test_dit_wide_mlp_vs_oracle(gpu, F, B, T, products):
+    """MLPs whose FF0 outgrows one round of the few-row tiles: both tile widths of the tiled
+    kernel's GELU (three products; 128 x 64 and, from 150 tiles, 128 x 128), the few-row kernel
+    past one tile per CU (six), and the first row past the fragment-order block."""
+    from larynx_amd.flow import DiTConfig
+    dit_vs_oracle(gpu, DiTConfig(depth=1, ff_inner=F), B, T, products)
 
 
 @pytest.fixture(scope="module")
