@@ -559,21 +559,6 @@ __global__ void wfrag_pack_kernel(const float* __restrict__ W, __bf16* __restric
   }
 }
 
-// Compute units of the current device (cached per device).
-int device_cus() {
-  static int cus[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cus[dev]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        n <= 0)
-      n = 256;
-    cus[dev] = n;
-  }
-  return cus[dev];
-}
-
 template <int EPI, int BMB, int OUT, int NP, int AP>
 int launch_bx(const BxArgs& a, const EpiArgs& ep, hipStream_t stream) {
   auto kern = gemm_bx_kernel<EPI, BMB, OUT, NP, AP>;
@@ -619,6 +604,20 @@ int dispatch_bx(const BxArgs& a, int out, const EpiArgs& ep, hipStream_t s) {
 }
 
 }  // namespace
+
+int device_cus() {
+  static int cus[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (!cus[dev]) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        n <= 0)
+      n = 256;
+    cus[dev] = n;
+  }
+  return cus[dev];
+}
 
 int bx_split_parts(int M, int N, int K, int bm) {
   // S: the most parts per split tile (at most 8, at most K / 64) with the split

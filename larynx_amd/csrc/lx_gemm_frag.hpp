@@ -26,8 +26,8 @@ struct FsArgs {
 };
 
 constexpr int kEpiNeox = 100;  // internal epilogue beside LX_EPI_*
-// Fewest 128 x 128 tiles (times K slices) that linear_ft runs as such, else 128 x 64
-// (M = 1000, N = 3072: 192 tiles 27.8 against 32.2 us; M = 256, N = 9728: 152 tiles
+// Fewest 128 x 128 tiles (times K slices) per 256 CUs that linear_ft runs as such, else 128
+// x 64 (M = 1000, N = 3072: 192 tiles 27.8 against 32.2 us; M = 256, N = 9728: 152 tiles
 // 25.5 / 31.3; M = 1000, N = 2048: 128 tiles 26.0 / 21.6).
 constexpr int kFtWideTiles = 150;
 

@@ -412,18 +412,18 @@ int dispatch_fs(FsArgs a, int out, const EpiArgs& ep, hipStream_t s) {
 // 3072 (768 of 64 x 64) 32.1 against 27.8 on the tiled kernel.
 template <int NP>
 bool pick_fs(const FsArgs& a, int out, const EpiArgs& ep, hipStream_t s, int* rc) {
-  const long nrb = (a.M + 31) / 32;
+  const long nrb = (a.M + 31) / 32, cus = device_cus();
   if (ep.kind == kEpiNeox) {
-    if (nrb * (a.N / 64) > 512) return false;
+    if (nrb * (a.N / 64) > 2 * cus) return false;
     FsArgs b = a;
     b.tiles_m = (int)nrb;
     b.tiles_n = a.N / 64;
     *rc = launch_fs<kEpiNeox, 1, 2, 4, FS_OUT_F32, NP, 1>(b, ep, s);
     return true;
   }
-  if (nrb * (a.N / 32) * a.slices <= 512)
+  if (nrb * (a.N / 32) * a.slices <= 2 * cus)
     *rc = dispatch_fs<1, 1, 4, NP, 1>(a, out, ep, s);
-  else if ((nrb + 1) / 2 * (a.N / 64) * a.slices <= 256)
+  else if ((nrb + 1) / 2 * (a.N / 64) * a.slices <= cus)
     *rc = dispatch_fs<2, 2, 4, NP, 1>(a, out, ep, s);
   else
     return false;
@@ -438,10 +438,10 @@ bool pick_fs(const FsArgs& a, int out, const EpiArgs& ep, hipStream_t s, int* rc
 // 1024, 200 rows, 336 tiles: 18.9 / 18.7).
 template <int NP, int AF>
 bool pick_fs_rows(const FsArgs& a, int out, const EpiArgs& ep, hipStream_t s, int* rc) {
-  const long nrb = (a.M + 31) / 32;
-  if (nrb * (a.N / 32) <= 256)
+  const long nrb = (a.M + 31) / 32, cus = device_cus();
+  if (nrb * (a.N / 32) <= cus)
     *rc = dispatch_fs<1, 1, 4, NP, AF>(a, out, ep, s);
-  else if (nrb * (a.N / 64) <= 256)
+  else if (nrb * (a.N / 64) <= cus)
     *rc = dispatch_fs<1, 2, 4, NP, AF>(a, out, ep, s);
   else
     return false;
@@ -476,7 +476,7 @@ bool linear_fs_rows(const lx_linear_bx& g, const EpiArgs& ep, hipStream_t stream
 // 24 1313 against 1296 us an evaluation) to one workgroup per CU.
 bool fs_takes_ln(int M, int N, int K, int products) {
   return products == 3 && K == kLnK && N % 64 == 0 && M > 64 &&
-         (long)((M + 31) / 32) * (N / 64) <= 256;
+         (long)((M + 31) / 32) * (N / 64) <= device_cus();
 }
 
 int linear_fs_ln(const FsLinear& g, const FsLn& ln, hipStream_t stream) {

@@ -249,7 +249,7 @@ int linear_ft(FsArgs a, int out, const EpiArgs& ep, int products, hipStream_t s)
                          : launch_ft<kEpiNeox, 1, 2, 2, FS_OUT_F32, 6>(a, ep, s);
   }
   tiles(2, 2);
-  if ((long)a.tiles_m * a.tiles_n * a.slices >= kFtWideTiles)
+  if ((long)a.tiles_m * a.tiles_n * a.slices >= kFtWideTiles * device_cus() / 256)
     return products == 3 ? dispatch_ft<2, 2, 3>(a, out, ep, s) : dispatch_ft<2, 2, 6>(a, out, ep, s);
   tiles(2, 1);
   return products == 3 ? dispatch_ft<2, 1, 3>(a, out, ep, s) : dispatch_ft<2, 1, 6>(a, out, ep, s);

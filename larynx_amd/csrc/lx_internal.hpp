@@ -16,6 +16,9 @@ inline size_t act_floats(size_t rows, size_t K, int parts) {
   return (rows + 31) / 32 * 32 * K * parts / 2;
 }
 
+// Compute units of the current device (cached per device; lx_gemm_bx.hip).
+int device_cus();
+
 // Device allocations of a composite object (lx_dit, lx_qwen2, lx_flow), made
 // at create time and released together when the object is destroyed.
 struct Arena {

@@ -62,7 +62,7 @@ int prefill_down_slices(int rows, int N, int K) {
   const int most = std::max(1, std::min(8, K / 512));
   const long fine = (long)((rows + 31) / 32) * (N / 32);
   const long wide = (long)((rows + 127) / 128) * (N / 128);
-  return (int)std::max<long>(1, std::min<long>(most, 256 / (rows <= 64 ? fine : wide)));
+  return (int)std::max<long>(1, std::min<long>(most, device_cus() / (rows <= 64 ? fine : wide)));
 }
 
 }  // namespace
@@ -278,7 +278,7 @@ int prefill_layer_frag(lx_qwen2* m, Layer& L, int rows, const float* next_norm, 
   o.K = H;
   LX_TRY(linear_fs(o, s));
   const long wide = (rows + 127) / 128;
-  if (m->products == 3 && wide * (2 * m->I / 128) > 256 && rows <= 1024 &&
+  if (m->products == 3 && wide * (2 * m->I / 128) > device_cus() && rows <= 1024 &&
       wide * 128 * 10 > (long)rows * 11) {
     LX_TRY(splitk_resid_rmsnorm(nullptr, 0, rows, H, nullptr, m->x, L.post_norm, m->eps, m->hn, s,
                                 LX_ACT_PACKED));
