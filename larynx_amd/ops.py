@@ -28,14 +28,14 @@ __all__ = [
 # torch.cuda.current_stream() builds a Stream object per call (2.8 us, most of the time a
 # 24-frame op spends in Python); the raw handle is the same stream at 0.2 us.  It is a private
 # name of torch: without it the public one serves.
-_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream",
+                      lambda device: torch.cuda.current_stream().cuda_stream)
+_device = torch.cuda.current_device
 
 
 def stream():
     """hipStream_t handle of torch's current stream."""
-    if _raw_stream is None:
-        return C.c_void_p(torch.cuda.current_stream().cuda_stream)
-    return C.c_void_p(_raw_stream(torch.cuda.current_device()))
+    return C.c_void_p(_raw_stream(_device()))
 
 
 def _p(t):

@@ -179,6 +179,7 @@ def test_ops_without_the_private_stream_getter():
     code = ("import types, torch\n"
             "if hasattr(torch._C, '_cuda_getCurrentRawStream'):\n"
             "    del torch._C._cuda_getCurrentRawStream\n"
+            "torch.cuda.current_device = lambda: 0\n"
             "from larynx_amd import ops\n"
             "torch.cuda.current_stream = lambda: types.SimpleNamespace(cuda_stream=4096)\n"
             "print(ops.stream().value)\n")
