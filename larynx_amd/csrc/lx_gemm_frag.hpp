@@ -35,7 +35,8 @@ constexpr int kFtWideTiles = 150;
 // checked) on the few-row kernel; the choice depends on the shape alone, so fp32 and
 // packed operands give the same bits.  false: not taken.
 bool linear_fs_rows(const lx_linear_bx& g, const EpiArgs& ep, hipStream_t stream, int* rc);
-int linear_ft(FsArgs a, int out, const EpiArgs& ep, int products, hipStream_t s);
+// Three products; outputs and epilogues as linear_fs, without the gated residual.
+int linear_ft(FsArgs a, int out, const EpiArgs& ep, hipStream_t s);
 
 __device__ __forceinline__ sbf16x8 frag_bf(uintx4_t v) { return __builtin_bit_cast(sbf16x8, v); }
 

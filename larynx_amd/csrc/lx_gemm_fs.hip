@@ -370,9 +370,13 @@ template <int RB, int CB, int KW, int NP, int AF>
 int dispatch_fs(FsArgs a, int out, const EpiArgs& ep, hipStream_t s) {
   a.tiles_m = (a.M + 32 * RB - 1) / (32 * RB);
   a.tiles_n = a.N / (32 * CB);
+  // 64 x 64 tiles of fragment-order operands: no gated residual and, with six products,
+  // no residual or partials (pick_fs)
+  constexpr bool GATED = AF != kAFrag || RB == 1, RESID = GATED || NP == 3;
   if constexpr (AF == kAFrag) {
-    if (out == FS_OUT_PARTIAL)
-      return launch_fs<LX_EPI_NONE, RB, CB, KW, FS_OUT_PARTIAL, NP, AF>(a, ep, s);
+    if constexpr (RESID)
+      if (out == FS_OUT_PARTIAL)
+        return launch_fs<LX_EPI_NONE, RB, CB, KW, FS_OUT_PARTIAL, NP, AF>(a, ep, s);
     if (out == FS_OUT_FRAG) {
       if (ep.kind == LX_EPI_GELU_TANH)
         return launch_fs<LX_EPI_GELU_TANH, RB, CB, KW, FS_OUT_FRAG, NP, AF>(a, ep, s);
@@ -397,8 +401,13 @@ int dispatch_fs(FsArgs a, int out, const EpiArgs& ep, hipStream_t s) {
     case LX_EPI_ROPE_PARTIAL:
       return launch_fs<LX_EPI_ROPE_PARTIAL, RB, CB, KW, FS_OUT_F32, NP, AF>(a, ep, s);
     case LX_EPI_GATED_RESID:
-      return launch_fs<LX_EPI_GATED_RESID, RB, CB, KW, FS_OUT_F32, NP, AF>(a, ep, s);
-    case LX_EPI_RESID: return launch_fs<LX_EPI_RESID, RB, CB, KW, FS_OUT_F32, NP, AF>(a, ep, s);
+      if constexpr (GATED)
+        return launch_fs<LX_EPI_GATED_RESID, RB, CB, KW, FS_OUT_F32, NP, AF>(a, ep, s);
+      break;
+    case LX_EPI_RESID:
+      if constexpr (RESID)
+        return launch_fs<LX_EPI_RESID, RB, CB, KW, FS_OUT_F32, NP, AF>(a, ep, s);
+      break;
     default: break;
   }
   set_error("linear_fs: epilogue kind %d not available", ep.kind);
@@ -409,21 +418,27 @@ int dispatch_fs(FsArgs a, int out, const EpiArgs& ep, hipStream_t s) {
 // CU; past that (false) the tiled kernel, whose wide tiles re-read W less often.
 // With cold weights, M = 148, N = 3072, K = 1024 (480 tiles) 12.7 us against 16.0 on
 // gemm_bx_kernel; M = 300, N = 3072 (240 of 64 x 64) 14.9 against 17.6; M = 1000, N =
-// 3072 (768 of 64 x 64) 32.1 against 27.8 on the tiled kernel.
+// 3072 (768 of 64 x 64) 32.1 against 27.8 on the tiled kernel.  Six products come with few
+// rows only and stay here at any tile count (FF0 of F = 8192, 150 rows, 384 tiles: an
+// evaluation of four blocks 604 -> 592 us against 128 x 64 tiled ones).  The gated residual
+// (N = 1024, at most 512 rows: two 32 x 32 tiles per CU) and, with six products, the residual
+// and the partials (the LM's o_proj and down_proj of at most 64 rows) keep 32 x 32 tiles.
 template <int NP>
 bool pick_fs(const FsArgs& a, int out, const EpiArgs& ep, hipStream_t s, int* rc) {
   const long nrb = (a.M + 31) / 32, cus = device_cus();
   if (ep.kind == kEpiNeox) {
-    if (nrb * (a.N / 64) > 2 * cus) return false;
+    if (NP == 3 && nrb * (a.N / 64) > 2 * cus) return false;
     FsArgs b = a;
     b.tiles_m = (int)nrb;
     b.tiles_n = a.N / 64;
     *rc = launch_fs<kEpiNeox, 1, 2, 4, FS_OUT_F32, NP, 1>(b, ep, s);
     return true;
   }
-  if (nrb * (a.N / 32) * a.slices <= 2 * cus)
+  const bool fine = ep.kind == LX_EPI_GATED_RESID ||
+                    (NP == 6 && (out == FS_OUT_PARTIAL || ep.kind == LX_EPI_RESID));
+  if (fine || nrb * (a.N / 32) * a.slices <= 2 * cus)
     *rc = dispatch_fs<1, 1, 4, NP, 1>(a, out, ep, s);
-  else if ((nrb + 1) / 2 * (a.N / 64) * a.slices <= cus)
+  else if (NP == 6 || (nrb + 1) / 2 * (a.N / 64) * a.slices <= cus)
     *rc = dispatch_fs<2, 2, 4, NP, 1>(a, out, ep, s);
   else
     return false;
@@ -557,7 +572,7 @@ int linear_fs(const FsLinear& g, hipStream_t stream) {
   int rc = LX_OK;
   if (g.products == 3 ? pick_fs<3>(a, g.out, ep, stream, &rc) : pick_fs<6>(a, g.out, ep, stream, &rc))
     return rc;
-  return linear_ft(a, g.out, ep, g.products, stream);
+  return linear_ft(a, g.out, ep, stream);
 }
 
 }  // namespace lx

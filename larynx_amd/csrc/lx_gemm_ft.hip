@@ -22,10 +22,10 @@
 namespace lx {
 namespace {
 
-template <int EPI, int RB, int CB, int KSL, int OUT, int NP>
+template <int EPI, int RB, int CB, int KSL, int OUT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 gemm_ft_kernel(FsArgs a, EpiArgs ep) {
-  constexpr int NPL = NP == 6 ? 3 : 2;
+  constexpr int NP = 3, NPL = 2;
   constexpr int CA = 2 * RB * KSL * NPL, CW = 2 * CB * KSL * NPL;  // 1 KB chunks per slab
   constexpr int LA = CA / 4, LW = CW / 4;                          // per wave
   static_assert(LA * 4 == CA && LW * 4 == CW, "chunks split evenly over the waves");
@@ -82,8 +82,7 @@ gemm_ft_kernel(FsArgs a, EpiArgs ep) {
 #pragma unroll
     for (int j = 0; j < LW; ++j) d[(CA + wave * LW + j) * 64] = gw[j];
   };
-  constexpr int kPa6[6] = {2, 1, 0, 1, 0, 0}, kPw6[6] = {0, 1, 2, 0, 1, 0};
-  constexpr int kPa3[3] = {1, 0, 0}, kPw3[3] = {0, 1, 0};
+  constexpr int kPa[NP] = {1, 0, 0}, kPw[NP] = {0, 1, 0};
   floatx16 acc[RB][CB];
 #pragma unroll
   for (int b = 0; b < RB; ++b)
@@ -114,19 +113,16 @@ gemm_ft_kernel(FsArgs a, EpiArgs ep) {
 #pragma unroll
         for (int c = 0; c < CB; ++c)
           acc[i][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              frag_bf(f.w[c][NP == 6 ? kPw6[q] : kPw3[q]]),
-              frag_bf(f.a[i][NP == 6 ? kPa6[q] : kPa3[q]]), acc[i][c], 0, 0, 0);
+              frag_bf(f.w[c][kPw[q]]), frag_bf(f.a[i][kPa[q]]), acc[i][c], 0, 0, 0);
   };
   static_assert(KSL == 2, "two k steps per slab");
   constexpr int NM = NP * RB * CB, NR = NPL * (RB + CB), NL = LA + LW;
-  // staging register sets (slab t in set t % NST): with six products a slab's
-  // MFMAs cover a load by themselves and a second set would spill
-  constexpr int NST = NP == 6 ? 1 : 2;
+  constexpr int NST = 2;  // staging register sets: slab t in set t % NST
   const int last = s1 - 1;
   uintx4_t ga[NST][LA], gw[NST][LW];
   Frag f0, f1;
   load(ga[0], gw[0], s0);
-  if (NST == 2) load(ga[NST - 1], gw[NST - 1], min(s0 + 1, last));
+  load(ga[1], gw[1], min(s0 + 1, last));
   store(ga[0], gw[0], 0);
   load(ga[0], gw[0], min(s0 + NST, last));
   __syncthreads();
@@ -201,12 +197,11 @@ gemm_ft_kernel(FsArgs a, EpiArgs ep) {
   }
 }
 
-template <int EPI, int RB, int CB, int KSL, int OUT, int NP>
+template <int EPI, int RB, int CB, int KSL, int OUT>
 int launch_ft(const FsArgs& a, const EpiArgs& ep, hipStream_t s) {
-  constexpr int NPL = NP == 6 ? 3 : 2;
-  auto kern = gemm_ft_kernel<EPI, RB, CB, KSL, OUT, NP>;
+  auto kern = gemm_ft_kernel<EPI, RB, CB, KSL, OUT>;
   static LdsLimit once;
-  const size_t lds = (size_t)2 * 2 * (RB + CB) * KSL * NPL * 1024;
+  const size_t lds = (size_t)2 * 2 * (RB + CB) * KSL * 2 * 1024;
   int rc = raise_lds_limit((const void*)kern, lds, once, "linear_ft");
   if (rc) return rc;
   hipLaunchKernelGGL(kern, dim3((unsigned)(a.tiles_m * a.tiles_n * a.slices)), dim3(256), lds, s,
@@ -214,45 +209,41 @@ int launch_ft(const FsArgs& a, const EpiArgs& ep, hipStream_t s) {
   return check_launch("gemm_ft_kernel");
 }
 
-template <int RB, int CB, int NP>
+template <int RB, int CB>
 int dispatch_ft(const FsArgs& a, int out, const EpiArgs& ep, hipStream_t s) {
-  if (out == FS_OUT_PARTIAL) return launch_ft<LX_EPI_NONE, RB, CB, 2, FS_OUT_PARTIAL, NP>(a, ep, s);
+  if (out == FS_OUT_PARTIAL) return launch_ft<LX_EPI_NONE, RB, CB, 2, FS_OUT_PARTIAL>(a, ep, s);
   if (out == FS_OUT_FRAG) {
     if (ep.kind == LX_EPI_GELU_TANH)
-      return launch_ft<LX_EPI_GELU_TANH, RB, CB, 2, FS_OUT_FRAG, NP>(a, ep, s);
-    return launch_ft<LX_EPI_SWIGLU_PAIRED, RB, CB, 2, FS_OUT_FRAG, NP>(a, ep, s);
+      return launch_ft<LX_EPI_GELU_TANH, RB, CB, 2, FS_OUT_FRAG>(a, ep, s);
+    return launch_ft<LX_EPI_SWIGLU_PAIRED, RB, CB, 2, FS_OUT_FRAG>(a, ep, s);
   }
-  switch (ep.kind) {
-    case LX_EPI_ROPE_PARTIAL:
-      return launch_ft<LX_EPI_ROPE_PARTIAL, RB, CB, 2, FS_OUT_F32, NP>(a, ep, s);
-    case LX_EPI_GATED_RESID:
-      return launch_ft<LX_EPI_GATED_RESID, RB, CB, 2, FS_OUT_F32, NP>(a, ep, s);
-    case LX_EPI_RESID: return launch_ft<LX_EPI_RESID, RB, CB, 2, FS_OUT_F32, NP>(a, ep, s);
-    default: break;
-  }
+  if (ep.kind == LX_EPI_RESID) return launch_ft<LX_EPI_RESID, RB, CB, 2, FS_OUT_F32>(a, ep, s);
   set_error("linear_ft: epilogue kind %d not available", ep.kind);
   return LX_ERR_ARG;
 }
 
 }  // namespace
 
-// Tiles of 128 x 128 or 128 x 64 (kFtWideTiles); the LM's q|k|v takes 64 x 128, a head
-// per wave.
-int linear_ft(FsArgs a, int out, const EpiArgs& ep, int products, hipStream_t s) {
+// Tiles of 128 x 128 or 128 x 64 (kFtWideTiles).  The LM's q|k|v takes 64 x 128, a head per
+// wave; the estimator's rotary q|k|v 128 x 64 (at most 512 rows: 96 tiles of 128 x 128).
+int linear_ft(FsArgs a, int out, const EpiArgs& ep, hipStream_t s) {
   auto tiles = [&](int rb, int cb) {
     a.tiles_m = (a.M + 64 * rb - 1) / (64 * rb);
     a.tiles_n = a.N / (64 * cb);
   };
   if (ep.kind == kEpiNeox) {
     tiles(1, 2);
-    return products == 3 ? launch_ft<kEpiNeox, 1, 2, 2, FS_OUT_F32, 3>(a, ep, s)
-                         : launch_ft<kEpiNeox, 1, 2, 2, FS_OUT_F32, 6>(a, ep, s);
+    return launch_ft<kEpiNeox, 1, 2, 2, FS_OUT_F32>(a, ep, s);
+  }
+  if (ep.kind == LX_EPI_ROPE_PARTIAL) {
+    tiles(2, 1);
+    return launch_ft<LX_EPI_ROPE_PARTIAL, 2, 1, 2, FS_OUT_F32>(a, ep, s);
   }
   tiles(2, 2);
   if ((long)a.tiles_m * a.tiles_n * a.slices >= kFtWideTiles * device_cus() / 256)
-    return products == 3 ? dispatch_ft<2, 2, 3>(a, out, ep, s) : dispatch_ft<2, 2, 6>(a, out, ep, s);
+    return dispatch_ft<2, 2>(a, out, ep, s);
   tiles(2, 1);
-  return products == 3 ? dispatch_ft<2, 1, 3>(a, out, ep, s) : dispatch_ft<2, 1, 6>(a, out, ep, s);
+  return dispatch_ft<2, 1>(a, out, ep, s);
 }
 
 }  // namespace lx

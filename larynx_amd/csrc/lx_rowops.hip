@@ -364,8 +364,8 @@ int adaln_resid(float* h, const float* partials, int splits, long partial_stride
                              gate_stride % 4 == 0),
              "adaln_resid: bad partials / gate");
   LX_REQUIRE(splits > 0 || y, "adaln_resid: nothing to do");
-  LX_REQUIRE(out_form < LX_ACT_FRAG2 || (D % 16 == 0 && splits == 0),
-             "adaln_resid: fragment order needs D %% 16 and no partials");
+  LX_REQUIRE(out_form < LX_ACT_FRAG2 || (D % 16 == 0 && D <= 4 * 256 && splits == 0),
+             "adaln_resid: fragment order needs D %% 16, D <= 1024 and no partials");
   LX_REQUIRE((mod_stride == 0 || mod_stride >= D) && mod_stride % 4 == 0,
              "adaln_resid: bad mod_stride %ld", mod_stride);
   LX_REQUIRE(((uintptr_t)h | (uintptr_t)y | (uintptr_t)shift | (uintptr_t)scale |
@@ -389,12 +389,8 @@ int adaln_resid(float* h, const float* partials, int splits, long partial_stride
   hipLaunchKernelGGL((adaln_resid_kernel<NVV, SM, ##__VA_ARGS__>), dim3(nblk), dim3(kRowsPerBlock * kWave), lds,     \
                      stream, h, partials, splits, partial_stride, bias, gate, gate_stride, shift, \
                      scale, mod_stride, y, rows, T, D, eps, out_form, gpb)
-  if (out_form >= LX_ACT_FRAG2 && nv <= 4)
+  if (out_form >= LX_ACT_FRAG2)
     LX_AR(4, 0, true);
-  else if (out_form >= LX_ACT_FRAG2 && nv <= 8)
-    LX_AR(8, 0, true);
-  else if (out_form >= LX_ACT_FRAG2)
-    LX_AR(16, 0, true);
   else if (nv <= 4 && splits <= 2)
     LX_AR(4, 2);
   else if (nv <= 4)
