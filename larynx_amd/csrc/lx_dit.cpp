@@ -38,7 +38,7 @@ constexpr float kRopeBase = 10000.0f;  // ROPE_FREQ_BASE (src/flow/internal.h:35
 constexpr int kRotDim = 64;        // ROT_DIM (src/flow/internal.h:25)
 constexpr int kProjSplitMax = 9;   // K slices of the proj_out split-K (gemm_splitk_plan's cap)
 constexpr int kSolveChunk = 16;    // solve steps whose modulations one GEMV computes
-// From frag_rows() (below) up to this many rows (B * T) the out and FF2 projections
+// From frag_block()'s limit (below) up to this many rows (B * T) the out and FF2 projections
 // run as two K slices whose sum is folded into the next modulated LayerNorm: at B * T = 1000 their
 // 64-row tiles number 128, half the CUs.
 constexpr int kPartialRows = 1024;
@@ -46,17 +46,17 @@ constexpr int kPartialRows = 1024;
 // with three and with six products.  One evaluation at B = 2: T = 24 2014 -> 1296
 // us, T = 74 1985 -> 1303, T = 160 2168 -> 1816, T = 256 2195 -> 2033 (T = 300 2368 /
 // 2389: even, and the larger launches keep the split tail); six products T = 24
-// 2413 -> 1602, T = 160 2573 -> 2422, T = 211 (422 rows) slower.  With an MLP wider than
-// kFragMlp FF0 outgrows one round of the CUs and FF2's K walk grows with it, and the split
-// tail is ahead sooner (four blocks, F = 4096, B = 2: three products T = 160 467 -> 430 us
-// but T = 161 445 -> 460; six T = 128 597 -> 491 but T = 129 570 -> 619; F = 3072 and 8192
-// alike).
-constexpr int kFragRows3 = 512, kFragRows3Wide = 320;
-constexpr int kFragRows6 = 320, kFragRows6Wide = 256;
-constexpr int kFragMlp = 2048;
-int frag_rows(int products, int F) {
-  if (products == 3) return F <= kFragMlp ? kFragRows3 : kFragRows3Wide;
-  return F <= kFragMlp ? kFragRows6 : kFragRows6Wide;
+// 2413 -> 1602, T = 160 2573 -> 2422, T = 211 (422 rows) slower.  Where FF0's 64 x 64 tiles
+// number more than one per CU the split tail is ahead sooner, past kFragRows*Any (four
+// blocks, B = 2: F = 4096, three products T = 160 467 -> 430 us but T = 161 445 -> 460; six T =
+// 128 597 -> 491 but T = 129 570 -> 619; F = 3072, whose FF0 fits at 320 rows, six T = 160 560 ->
+// 543).
+constexpr int kFragRows3 = 512, kFragRows3Any = 320;
+constexpr int kFragRows6 = 320, kFragRows6Any = 256;
+bool frag_block(int rows, int products, int F) {
+  const bool fits = (long)((rows + 63) / 64) * (F / 64) <= device_cus();
+  if (products == 3) return rows <= (fits ? kFragRows3 : kFragRows3Any);
+  return rows <= (fits ? kFragRows6 : kFragRows6Any);
 }
 
 }  // namespace
@@ -185,9 +185,9 @@ int forward_core(lx_dit* m, const float* x, long x_bstride, const float* mu, con
     const float* gate = nullptr;
   } pend;
   bool pending = false;
-  const bool fs = m->frag && rows <= frag_rows(m->products, m->F);
+  const bool fs = m->frag && frag_block(rows, m->products, m->F);
   const bool partial = m->frag && !fs && rows <= kPartialRows;
-  // Up to frag_rows() rows every GEMM input of the block (the modulated
+  // Where frag_block() holds every GEMM input of the block (the modulated
   // LayerNorms' output, attention's output, FF0's GELU output) is written by its
   // producer in fragment order, two parts for three products and three for six,
   // and the residual goes in by the out / FF2 epilogues.  Past them three products

@@ -43,7 +43,7 @@ def test_dit_projection_tiles_vs_oracle(gpu, B, T, products):
 
 
 @pytest.mark.parametrize("F,B,T,products", [
-    (4096, 2, 37, 6), (4096, 1, 320, 3), (4096, 1, 321, 3), (4096, 2, 128, 6), (4096, 1, 257, 6),
+    (4096, 2, 37, 6), (4096, 1, 320, 3), (4096, 1, 321, 3), (4096, 2, 128, 6), (4096, 1, 257, 6), (3072, 1, 320, 6),
     (8192, 1, 149, 3), (8192, 1, 289, 3), (8192, 2, 75, 6),
 ])
 def test_dit_wide_mlp_vs_oracle(gpu, F, B, T, products):
