@@ -1,7 +1,8 @@
 """The projections on fragment-order activations (lx_gemm_fs.hip, lx_gemm_ft.hip) through the
 estimator and the Qwen2 prefill, against the oracle at the row counts where a launch changes
 its tiles: part of one 32-row block, whole blocks and one row past them, the last row count of
-the 32 x 32 and 64 x 64 tiles, and the first past the fragment-order block."""
+the 32 x 32 and 64 x 64 tiles, the tiled kernel's three tile shapes, and the first row past the
+fragment-order block."""
 import numpy as np
 import pytest
 import torch
@@ -54,17 +55,47 @@ def test_dit_wide_mlp_vs_oracle(gpu, F, B, T, products):
     dit_vs_oracle(gpu, DiTConfig(depth=1, ff_inner=F), B, T, products)
 
 
-@pytest.fixture(scope="module")
-def qwen2(gpu):
+def make_lm(gpu, n_layers, max_ctx):
     from larynx_amd.llm import Qwen2Config, Qwen2LM, qwen2_param_shapes
-    cfg = Qwen2Config(n_layers=2, text_vocab=2000)
+    cfg = Qwen2Config(n_layers=n_layers, text_vocab=2000)
     params = orc.make_params(qwen2_param_shapes(cfg), 78)
     for k in params:
         if k.endswith("layernorm.weight") or k == "norm.weight":
             params[k] = (params[k] + 1.0).astype(np.float32)
-    lm = Qwen2LM({k: torch.from_numpy(v).to(gpu) for k, v in params.items()}, cfg, max_ctx=1100)
+    lm = Qwen2LM({k: torch.from_numpy(v).to(gpu) for k, v in params.items()}, cfg, max_ctx=max_ctx)
+    return cfg, params, lm
+
+
+@pytest.fixture(scope="module")
+def qwen2(gpu):
+    cfg, params, lm = make_lm(gpu, 2, 1100)
     yield cfg, params, lm
     lm.close()
+
+
+@pytest.fixture(scope="module")
+def qwen2_long(gpu):
+    cfg, params, lm = make_lm(gpu, 1, 2750)
+    yield cfg, params, lm
+    lm.close()
+
+
+def prefill_vs_oracle(gpu, model, L, products):
+    cfg, params, lm = model
+    announce(f"qwen2 prefill L={L} products={products}")
+    lm.set_products(products)
+    lm_in = torch.from_numpy(orc.normal((L, cfg.hidden), 500 + L, 1, 0.5)).to(gpu)
+    logits, hidden, final = lm.prefill(lm_in, capture=True)
+    torch.cuda.synchronize()
+    o = orc.Qwen2(params, cfg, cap=L)
+    rl, rh, rf = o.prefill(lm_in.cpu().numpy(), capture=True)
+    tol = 5e-5 if products == 3 else 1e-5
+    for layer in range(cfg.n_layers):
+        assert orc.rel_err(hidden[layer].cpu().numpy(), rh[layer]) < tol, layer
+        k, v = lm.cache_views(layer)
+        assert orc.rel_err(k[:L].cpu().numpy(), o.k_cache[layer, :L]) < tol, layer
+        assert orc.rel_err(v[:L].cpu().numpy(), o.v_cache[layer, :L]) < tol, layer
+    assert orc.rel_err(logits.cpu().numpy(), rl) < tol
 
 
 @pytest.mark.parametrize("L,products", [
@@ -74,21 +105,14 @@ def qwen2(gpu):
 def test_prefill_projection_tiles_vs_oracle(gpu, qwen2, L, products):
     """q|k|v with the rotary and cache append in its epilogue, o_proj's residual epilogue,
     gate/up with SwiGLU in fragment order and down_proj's K slices."""
-    cfg, params, lm = qwen2
-    announce(f"qwen2 prefill L={L} products={products}")
-    lm.set_products(products)
-    lm_in = torch.from_numpy(orc.normal((L, cfg.hidden), 500 + L, 1, 0.5)).to(gpu)
-    logits, hidden, final = lm.prefill(lm_in, capture=True)
-    torch.cuda.synchronize()
-    o = orc.Qwen2(params, cfg, cap=1100)
-    rl, rh, rf = o.prefill(lm_in.cpu().numpy(), capture=True)
-    tol = 5e-5 if products == 3 else 1e-5
-    for layer in range(cfg.n_layers):
-        assert orc.rel_err(hidden[layer].cpu().numpy(), rh[layer]) < tol, layer
-        k, v = lm.cache_views(layer)
-        assert orc.rel_err(k[:L].cpu().numpy(), o.k_cache[layer, :L]) < tol, layer
-        assert orc.rel_err(v[:L].cpu().numpy(), o.v_cache[layer, :L]) < tol, layer
-    assert orc.rel_err(logits.cpu().numpy(), rl) < tol
+    prefill_vs_oracle(gpu, qwen2, L, products)
+
+
+@pytest.mark.parametrize("L", [1152, 1153, 2435, 2689, 2750])
+def test_prefill_long_tiles_vs_oracle(gpu, qwen2_long, L):
+    """The last length of o_proj on the few-row kernel, its 128 x 64 (1153-2688 rows) and 128 x
+    128 tiles, and down_proj whole in K on 128 x 64 (2305-2688 rows) and 128 x 128 ones."""
+    prefill_vs_oracle(gpu, qwen2_long, L, 3)
 
 
 @pytest.mark.parametrize("M,N,K,products,lda", [

@@ -32,6 +32,14 @@ def qwen(gpu):
     lm.close()
 
 
+@pytest.fixture
+def products_of(qwen):
+    """Sets the shared LM's product count for one test."""
+    lm = qwen[3]
+    yield lm.set_products
+    lm.set_products(3)
+
+
 def test_prefill_then_decode(gpu, qwen):
     cfg, params, _, lm = qwen
     rng = np.random.default_rng(5)
@@ -200,15 +208,15 @@ def test_decode_crosses_split_classes(gpu, qwen, max_ctx, n0):
     graph.close()
 
 
-@pytest.mark.parametrize("L", [1, 37, 200, 300])
-def test_prefill_ragged_lengths(gpu, qwen, L):
-    """Prefill at lengths that leave partial 64-row tiles and change the
-    split-K plan (1 row: one tile per column band; 300 rows: five bands).  At
-    200 and 300 rows the gate/up launch runs the split tail on 64-row tiles (4
-    row bands x 76 column tiles = 256 whole + 48 in five k ranges; 5 x 76 = 256
-    whole + 124 in two), with the last row band partial."""
+@pytest.mark.parametrize("L,products", [(1, 3), (37, 3), (200, 3), (300, 3), (200, 6), (300, 6)])
+def test_prefill_ragged_lengths(gpu, qwen, products_of, L, products):
+    """Prefill at lengths that leave partial row tiles and change the K slices of
+    down_proj.  With six products at 200 and 300 rows the gate/up launch runs the
+    split tail on 64-row tiles (4 row bands x 76 column tiles = 256 whole + 48 in
+    five k ranges; 5 x 76 = 256 whole + 124 in two), with the last row band partial."""
+    products_of(products)
     cfg, params, _, lm = qwen
-    announce(f"qwen2 prefill L={L}")
+    announce(f"qwen2 prefill L={L} products={products}")
     lm_in = torch.from_numpy(orc.normal((L, cfg.hidden), 300 + L, 1, 0.5)).to(gpu)
     logits, hidden, final = lm.prefill(lm_in, capture=True)
     torch.cuda.synchronize()
@@ -225,13 +233,15 @@ def test_prefill_ragged_lengths(gpu, qwen, L):
         assert orc.rel_err(v[:L].cpu().numpy(), o.v_cache[layer, :L]) < TOL
 
 
-def test_prefill_split_tail_is_deterministic(gpu, qwen):
-    """The gate/up launch at L=256 (split tail: 256 whole tiles, 48 in five k
-    ranges) sums the parts of its split tiles in k order whichever part arrives
-    last: two prefills of the same input give bit-identical hidden states,
-    logits and caches."""
+@pytest.mark.parametrize("products", [6, 3])
+def test_prefill_split_tail_is_deterministic(gpu, qwen, products_of, products):
+    """Two prefills of the same input give bit-identical hidden states, logits and
+    caches.  With six products the gate/up launch at L=256 runs the split tail (256
+    whole tiles, 48 in five k ranges) and sums the parts of its split tiles in k
+    order whichever part arrives last; three products run the fragment-order layer."""
     cfg, params, _, lm = qwen
-    announce("qwen2 prefill L=256 twice (split tail determinism)")
+    products_of(products)
+    announce(f"qwen2 prefill L=256 twice, products={products}")
     lm_in = torch.from_numpy(orc.normal((256, cfg.hidden), 4040, 1, 0.5)).to(gpu)
     runs = []
     for _ in range(2):
