@@ -312,15 +312,26 @@ int lx_wfrag_pack_f32(const float* W, void* Wf, int N, int K, hipStream_t stream
 int lx_linear_bx_f32(const lx_linear_bx* g, hipStream_t stream);
 
 /* Scaled-dot-product attention (flash-style, scores never stored; fp32
- * arithmetic, on the fp32 matrix cores or, for grids that fill the CUs in whole
- * rounds, on the bf16 ones with every operand split into three bf16 parts and
- * six exact partial products accumulated in fp32):
+ * arithmetic, on the fp32 matrix cores or on the bf16 ones, the split kernel,
+ * with every operand split into three bf16 parts and six exact partial
+ * products accumulated in fp32, an error at the fp32 kernel's level):
  *   o[b, t, h*hd:(h+1)*hd] = softmax(scale * q_h k_g^T [+ causal mask]) v_g
  * with g = h / (n_heads / n_kv_heads) (GQA, consecutive like HF repeat_kv).
  * q: (B, Tq, *) row stride ldq, head h at column h*hd; k, v: (B, Tk, *) row
  * strides ldk/ldv, kv head g at column g*hd; o: (B, Tq, *) row stride ldo.
  * causal != 0: query i (absolute position q_offset + i) sees keys <= that
  * position.  head_dim must be 64.
+ * Which kernel runs depends on the grid, W(n) = ceil(Tq / n) * n_heads * B
+ * workgroups of n queries:
+ *   W(64) < 256       fp32 while W(32) <= 256 (causal: W(64) < 176), else split;
+ *   W(128) a multiple of 256, or W(64) == 256      split;
+ *   other grids       fp32, causal ones split.
+ * On the split kernel an infinite or NaN element, or a finite one above
+ * 3.3895e38 in magnitude (k and v; q after its scaling), makes NaN of the query
+ * that holds it in q, and of every query of that head that sees its key in k or
+ * v (causal: also undefined for the queries before a v element's key), where
+ * the fp32 kernel gives what fp32 sums give for infinities; NaN inputs are
+ * undefined there.
  * Replaces attention() (src/flow/dit.cpp:34-51; src/llm/ops.cpp:49-65) and
  * repeat_kv (src/llm/ops.cpp:32-47). */
 int lx_attention_f32(const float* q, int ldq, const float* k, int ldk, const float* v,
@@ -329,7 +340,9 @@ int lx_attention_f32(const float* q, int ldq, const float* k, int ldk, const flo
                      hipStream_t stream);
 /* lx_attention_f32 with the split-operand kernel's product count: 6 (as
  * lx_attention_f32) or 3 (two bf16 parts per operand, three products: about
- * half the matrix-core work; the grids that run the fp32 kernel ignore it).
+ * half the matrix-core work).  With 3 every grid of W(64) >= 256 runs the split
+ * kernel with three products; smaller ones run as with 6 (at B = 2 and 16
+ * heads six products for Tq 257-448, the fp32 kernel below).
  * out_packed != 0: o receives two-part packed rows (lx_linear_bx's a_packed
  * operand) instead of fp32.  kv_packed != 0: k and v are two-part packed rows
  * (lx_linear_bx's LX_BX_OUT_PACKED), for three products on the layouts of the

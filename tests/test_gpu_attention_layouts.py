@@ -44,3 +44,32 @@ def test_attention_layouts(gpu, B, T, nh, nkv, products, causal, off, tol):
     ref = reference(q.double(), k.double(), v.double(), nh, nkv, causal, off)
     err = ((o - ref).norm() / ref.norm()).item()
     assert err < tol, err
+
+
+@pytest.mark.parametrize("B,T,nh,nkv,products,causal", [
+    (2, 300, 16, 16, 3, False), (2, 300, 16, 16, 6, False), (1, 800, 14, 2, 6, True),
+])
+def test_attention_nonfinite_where_six_products_replace_fp32(gpu, B, T, nh, nkv, products, causal):
+    """Grids under one 64-query workgroup per CU that run six products whatever the caller asks
+    for: an infinite q element makes its query NaN, an infinite k or v element every query that
+    sees its key (a later key's v also queries before it, undefined), as on the larger grids of
+    that kernel; the rest stays finite."""
+    from larynx_amd import ops
+    announce(f"attention non-finite B={B} T={T} products={products} causal={causal}")
+    g = torch.Generator().manual_seed(T)
+    q = torch.randn(B, T, nh, 64, generator=g)
+    k, v = (torch.randn(B, T, nkv, 64, generator=g) for _ in range(2))
+    q[0, 10, nh - 2, 5] = np.inf
+    k[B - 1, 20, nkv - 1, 7] = np.inf
+    v[0, 40, 0, 9] = -np.inf
+    rep = nh // nkv
+    hit, free = torch.zeros(B, T, nh, dtype=torch.bool), torch.zeros(B, T, nh, dtype=torch.bool)
+    hit[0, 10, nh - 2] = True
+    hit[B - 1, (20 if causal else 0):, nh - rep:] = True
+    vhit = torch.zeros(B, T, nh, 64, dtype=torch.bool)
+    vhit[0, (40 if causal else 0):, :rep, 9] = True
+    free[0, :, :rep] = True
+    o = ops.attention(*(x.flatten(2).to(gpu) for x in (q, k, v)), nh, nkv, causal=causal,
+                      products=products).cpu().view(B, T, nh, 64)
+    assert o[hit].isnan().all() and o[vhit].isnan().all()
+    assert o[~hit & ~free].isfinite().all()
