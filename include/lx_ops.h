@@ -262,10 +262,11 @@ int lx_linear_split_f32(const float* x, int ldx, const void* planes, const float
  * The last part of a split tile to finish sums the parts' products in k order
  * and applies the epilogue (deterministic, no waiting).  ws needs CUs * bm *
  * 128 floats, counters one per tile; other shapes run as without scratch.
- * Without scratch a call of few rows (at most one 32 x 64 tile per CU) runs a
- * kernel that splits K over a workgroup's waves, and one whose rows exceed one
- * 64-row tile per CU by less than half runs 96-row tiles; bm = 64 results are
- * the same for fp32 and packed operands either way.
+ * Without scratch a call of few rows (at most one 32 x 64 tile per CU, any
+ * epilogue but SWIGLU_PAIRED) runs a kernel that splits K over a workgroup's
+ * waves, and a bm = 64 one whose rows exceed one 64-row tile per CU by less than
+ * half runs 96-row tiles; bm = 64 results are the same for fp32 and packed
+ * operands either way.
  * products: 6 (or 0) forms each element pair as the six products of the
  * three-part splits (fp32-level error, the default); 3 uses two-part splits
  * (x0 + x1, 16 significant bits each) and the three products a0 b0 + a0 b1 +

@@ -571,8 +571,9 @@ int launch_bx(const BxArgs& a, const EpiArgs& ep, hipStream_t stream) {
   return check_launch("gemm_bx_kernel");
 }
 
-// Packed operands exist for three products (AP = 1 on 64- and 128-row tiles,
-// BX_OUT_PACKED on 64-row tiles; the host checks this).
+// Packed operands exist for three products (AP = 1 on every tile height, BX_OUT_PACKED
+// on 64- and 96-row tiles, both of which bm = 64 asks for; the host checks this).  96-row
+// tiles have no raw partials.
 template <int BMB, int NP, int AP = 0>
 int dispatch_bx(const BxArgs& a, int out, const EpiArgs& ep, hipStream_t s) {
   if constexpr (BMB != 3)

@@ -1,18 +1,22 @@
-// Split-operand GEMM for many rows: operands in MFMA fragment order, staged
-// through LDS in large tiles.
+// Split-operand GEMM past the few-row kernel's tiles (lx_gemm_fs.hip): operands in
+// MFMA fragment order, staged through LDS in large tiles.
 //
-// The arithmetic of gemm_bx_kernel (two or three bf16 parts per operand, three
-// or six products on v_mfma_f32_32x32x16_bf16, fp32 accumulation), for
-// activations written in fragment order by their producers (LX_ACT_FRAG*).
-// gemm_bx_kernel streams every wave's W columns from L2 and its 64 x 128 tiles
-// read 1.77 GB through L2 for q|k|v at B * T = 6000 (127 us, 14 TB/s: what the L2s
-// deliver).  Here 2 x 2 waves of (32 RB) x (32 CB) outputs share both operands in
-// LDS: tiles of 256 x 128 (RB = 4) or 128 x 128 (RB = 2) halve that traffic, and
-// 1 KB fragments go global -> registers -> LDS -> registers in lane order, with no
-// address arithmetic, split or bank conflict on the way.  Two workgroups share a
-// CU and cover each other's barriers.  W is the MFMA's A operand: a lane's
-// accumulator quad is four consecutive columns of one row, and the epilogue works
-// on float4 straight from the accumulators.
+// The arithmetic of gemm_bx_kernel with three products (two bf16 parts per operand,
+// v_mfma_f32_32x32x16_bf16, fp32 accumulation), for activations written in fragment
+// order by their producers (LX_ACT_FRAG2).  That kernel streams every wave's W columns
+// from L2 once per 64-row tile.  Here 2 x 2 waves of (32 RB) x (32 CB) outputs share
+// both operands in LDS, in tiles of 128 x 128, 128 x 64 or (the LM's q|k|v, a head per
+// wave) 64 x 128, and 1 KB fragments go global -> registers -> LDS -> registers in lane
+// order, with no address arithmetic, split or bank conflict on the way.  Two workgroups
+// (64 KB of LDS each at most) share a CU and cover each other's barriers.  W is the
+// MFMA's A operand: a lane's accumulator quad is four consecutive columns of one row,
+// and the epilogue works on float4 straight from the accumulators.
+//
+// It runs the LM prefill's gate/up past 64 rows, down_proj past 128, q|k|v past 896 and
+// o_proj past 1152, the estimator's q|k|v at 321-512 rows and FF0 of an MLP wider than
+// 2048.  With cold weights: gate/up L = 256 31.4 -> 25.7 us, L = 1531 99.9 -> 96.0; down_proj
+// L = 1531, three K slices, 63.7 -> 42.4.  Bound by LDS traffic (each wave reads both
+// operands' fragments from it) at one to two waves per SIMD.
 #include <algorithm>
 
 #include "lx_common.hpp"

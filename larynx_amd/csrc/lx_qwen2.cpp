@@ -188,10 +188,12 @@ int prefill_mlp(lx_qwen2* m, Layer& L, int rows, const float* next_norm, hipStre
   lx_epilogue swiglu{};
   swiglu.kind = LX_EPI_SWIGLU_PAIRED;
   if (m->frag) {
-    // gate/up + SwiGLU: 64-row tiles with the split tail where it applies (L =
-    // 256: 304 tiles, 256 whole and 48 in five k ranges; 24.3 vs 25.3 us on
-    // 128-row tiles with cold weights), else 128-row tiles while they fit one
-    // round over the CUs, else 64-row tiles (L = 1024: 95 vs 116 us)
+    // gate/up + SwiGLU: 64-row tiles with the split tail where it applies (six
+    // products L = 256: 304 tiles, 256 whole and 48 in five k ranges; 29.6 vs 39.7 us
+    // on 128-row tiles with cold weights), else 128-row tiles while they fit one
+    // round over the CUs, else 64-row tiles.  Three products come here with more
+    // 128-row tiles than CUs, which at this width (76 column tiles) is past the split
+    // tail's rows
     const bool split = bx_split_parts(rows, 2 * m->I, H, 64) > 0;
     lx_linear_bx g{};
     if (split) {
@@ -239,7 +241,9 @@ int prefill_mlp(lx_qwen2* m, Layer& L, int rows, const float* next_norm, hipStre
 // fragment order by its producer; the last norm is fp32 (the logits GEMM reads it).
 // Where 128-row tiles pad the rows by a tenth or more past one round of the CUs (L =
 // 400: 304 gate/up tiles, a quarter of their rows padding, 42.6 us against 36.9), the
-// MLP runs on the 64-row tiles of the split-operand GEMM instead.
+// MLP runs on the 64-row tiles of the split-operand GEMM instead, up to 1024 rows: with
+// more the padding costs less than that kernel's L2 traffic (whole prefill, L = 1040 4.18 ms
+// against 4.30 on 64-row tiles, L = 1160 4.51 / 5.13).
 int prefill_layer_frag(lx_qwen2* m, Layer& L, int rows, const float* next_norm, hipStream_t s,
                        bool last) {
   const int H = m->H, KV = m->KV, QKV = m->QKV;
