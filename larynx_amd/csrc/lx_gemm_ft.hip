@@ -15,8 +15,9 @@
 // It runs the LM prefill's gate/up past 64 rows, down_proj past 128, q|k|v past 896 and
 // o_proj past 1152, the estimator's q|k|v at 321-512 rows and FF0 of an MLP wider than
 // 2048.  With cold weights: gate/up L = 256 31.4 -> 25.7 us, L = 1531 99.9 -> 96.0; down_proj
-// L = 1531, three K slices, 63.7 -> 42.4.  Bound by LDS traffic (each wave reads both
-// operands' fragments from it) at one to two waves per SIMD.
+// L = 1531, three K slices, 63.7 -> 42.4.  Under counters the L = 1531 launches keep the
+// matrix pipe 0.52-0.54 and the LDS 0.36 busy at a clock of 1.7 GHz; at L = 256 (152 tiles,
+// one workgroup on 152 of 256 CUs) 0.24 and 0.17 at 2.0: a wave per SIMD waiting.
 #include <algorithm>
 
 #include "lx_common.hpp"
